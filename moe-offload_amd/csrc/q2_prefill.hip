@@ -4,30 +4,23 @@
 // rows sorted by expert, chunk-local slot = rank of the expert in the chunk),
 // prefill_qproj.py:18-40 (gather_qmm over the sorted rows), cpp/src/layers.cpp:364-600.
 // For the sorted rows r of segment u (one expert, weights = blob seg_slot[u] of the pool):
-//     h_r = silu(G_u x_r) * (U_u x_r)        (k_q2g_proj<.., kGateUp>, fp16 out)
-//     y_r = D_u h_r                          (k_q2g_proj<.., kDown>, fp16 out, row row_out[r])
+//     h_r = silu(G_u x_r) * (U_u x_r)        (fp16 out)
+//     y_r = D_u h_r                          (fp16 out, row row_out[r])
 // with W = scale * q + bias per group of 64 inputs (2-bit codes, 16 per u32, LSB first).
 //
-// Tiling.  The rows of a segment form M tiles of 16 (v_mfma_f32_16x16x32_f16), taken in
-// batches of up to 2 tiles.  A block of 4 waves works on one segment and one slice of weight
-// rows; each wave owns 4 subtiles of 16 weight rows (gate/up: 2 x 16 rows of each projection =
-// 128 intermediate rows per block; down: 4 x 16 = 256 output rows).  Per 256-wide K chunk j a
-// lane (n = lane & 15, kq = lane >> 4) loads group 4j + kq of weight row n (one 16-byte load of
-// 64 codes plus the (scale, bias) word), dequantises it once and multiplies it into every tile
-// of the batch; the chunk's activations of the batch's rows are staged in LDS (each thread
-// stages 2 units of 16 bytes per tile).  The next chunk's weights and activations are loaded
-// while the current chunk is multiplied.  The gate/up grid holds every (segment, slice) item
-// twice: segments of more than one batch run in the first half, so their blocks, the longest,
-// are dispatched before the rest.  At K = 2048 gate/up runs in the whole-K form instead
-// (k_q2g_gu_wk: per M tile, each wave's weight subtiles requested over the whole K at once, the
-// tile's activations staged once; the same two-pass grid, long segments first).  At K = 512 down
-// runs in the whole-K form as well (k_q2g_dn_wk: each wave's 4 subtiles loaded once over the whole
-// K and kept in registers while the segment's M tiles pass through LDS; two-pass grid).
+// Tiling.  The rows of a segment form M tiles of 16 (v_mfma_f32_16x16x32_f16).  k_q2g_mm takes up to
+// 64 rows of a segment per pass over its weights, with their activations staged in LDS for the whole
+// K and, for all but short calls, a fixed grid whose blocks split the work evenly.  With few rows per
+// expert, K = 2048 gate/up and K = 512 down run in the whole-K forms: k_q2g_gu_wk (per M tile, each
+// wave's weight subtiles requested over the whole K at once, the tile's activations staged once) and
+// k_q2g_dn_wk (each wave's 4 subtiles loaded once and kept in registers while the segment's M tiles
+// pass through LDS), both with a grid that holds every (segment, slice) item twice: segments of
+// several tiles run in the first half, so their blocks, the longest, are dispatched before the rest.
 //
 // Dequantisation.  A 2-bit code in the low bits of a nibble is the fp4 (e2m1) value q/2, so
 // w & 0x33333333 (even codes) and (w >> 2) & 0x33333333 (odd codes) are 8 fp4 values each;
-// v_cvt_scalef32_pk_f16_fp4 turns a byte into two exact halves, and one v_pk_fma_f16 with
-// (2*scale, bias) gives the fp16 weight scale*q + bias rounded once (MLX's dequantised weight).
+// v_cvt_scalef32_pk_f16_fp4 with scale 2 turns a byte into two exact halves q, and one v_pk_fma_f16
+// with (scale, bias) gives the fp16 weight scale*q + bias rounded once (MLX's dequantised weight).
 //
 // K order.  Inside an MFMA the K positions are permuted identically for A and B: the even codes
 // of a 32-bit word pair with activations [x0 x2 .. x14] of its 16 inputs and the odd codes with
@@ -39,6 +32,9 @@
 // fp16 is exact for the normal range of fp16).
 #include <hip/hip_fp16.h>
 
+#include <cstdlib>
+#include <type_traits>
+
 #include "moe_common.h"
 
 namespace {
@@ -48,7 +44,6 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMT = 16;          // rows per M tile
-constexpr int kSub = 4;          // 16-row weight subtiles per wave
 constexpr int kMaxChunks = 10;   // K <= 2560
 constexpr int kGateUp = 0, kDown = 1;
 
@@ -59,11 +54,15 @@ __device__ __forceinline__ int xcd_order(int b, int nb) {
     return x < rem ? x * (per + 1) + i : rem * (per + 1) + (x - rem) * per + i;
 }
 
-__device__ __forceinline__ f16x8 dequant8(uint32_t bits, f16x2 s2, f16x2 b2) {
-    f16x2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 1.0f, 0);
-    f16x2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 1.0f, 1);
-    f16x2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 1.0f, 2);
-    f16x2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 1.0f, 3);
+// Codes of one 32-bit word (8 of them: bits already masked to the low two bits of every nibble) ->
+// 8 fp16 weights scale * q + bias.  sb = (scale, bias) as one fp16 pair.
+__device__ __forceinline__ f16x8 dequant8(uint32_t bits, uint32_t sb) {
+    const f16x2 p = __builtin_bit_cast(f16x2, sb);
+    const f16x2 s2 = {p.x, p.x}, b2 = {p.y, p.y};
+    f16x2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 2.0f, 0);
+    f16x2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 2.0f, 1);
+    f16x2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 2.0f, 2);
+    f16x2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(bits, 2.0f, 3);
     a = __builtin_elementwise_fma(a, s2, b2);
     b = __builtin_elementwise_fma(b, s2, b2);
     c = __builtin_elementwise_fma(c, s2, b2);
@@ -93,14 +92,6 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// M tiles multiplied per pass over a segment's weights: 2 for both projections.  Gate/up: the
-// registers 4 tiles would hold leave no room for the next chunk's activations in flight (only
-// segments of more than 32 rows take a second pass; 128 us per 512-token chunk against 133 with
-// 4 tiles and the activations loaded after the multiply).  Down: a short K, every pass is two
-// chunks of dependent round trips (62 us at 2 tiles, 70 at 1 and at 4).
-template <int MODE>
-constexpr int max_mt() { return 2; }
-
 // One (scale, bias) fp16 word from two 16-bit values of the 9-tensor form.
 template <int SBF>
 __device__ __forceinline__ uint32_t sb_word(uint32_t sc, uint32_t bi) {
@@ -118,8 +109,8 @@ __device__ __forceinline__ uint32_t sb_word(uint32_t sc, uint32_t bi) {
 // first pair is multiplied.  The tile's activation rows are staged in LDS once for the whole K,
 // already split into the MFMA's even / odd input fragments: one barrier per tile, after which the
 // waves run independently.  A K position of an MFMA pairs lane group kq's group GPL*kq + i with
-// the same inputs on the A side; the even/odd code split inside a word is the one of k_q2g_proj.
-// Bit for bit this is not k_q2g_proj's sum order (another K order inside the MFMAs).
+// the same inputs on the A side; the even/odd code split inside a word is the one described above.
+// Bit for bit this is not k_q2g_mm's sum order (another K order inside the MFMAs).
 template <int GPL, int SBF>
 __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n_src_rows,
                                            const int32_t* __restrict__ row_map, int r0, int rows, int slot,
@@ -205,14 +196,6 @@ __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n
         const uint4* arow = a_lds + n * UPR;
 #pragma unroll
         for (int i = 0; i < GPL; ++i) {
-            f16x2 s2[2], b2[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const f16x2 sb = __builtin_bit_cast(f16x2, wd[h][i]);
-                const _Float16 two_s = sb.x * (_Float16)2.0f;
-                s2[h] = (f16x2){two_s, two_s};
-                b2[h] = (f16x2){sb.y, sb.y};
-            }
             const int u0 = 8 * (GPL * kq + i);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -223,8 +206,8 @@ __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n
                 for (int h = 0; h < 2; ++h) {
                     const uint4 cv = c[h][i];
                     const uint32_t wq = q == 0 ? cv.x : q == 1 ? cv.y : q == 2 ? cv.z : cv.w;
-                    const f16x8 b_ev = dequant8(wq & 0x33333333u, s2[h], b2[h]);
-                    const f16x8 b_od = dequant8((wq >> 2) & 0x33333333u, s2[h], b2[h]);
+                    const f16x8 b_ev = dequant8(wq & 0x33333333u, wd[h][i]);
+                    const f16x8 b_od = dequant8((wq >> 2) & 0x33333333u, wd[h][i]);
                     f32x4& acc = h ? accu : accg;
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_ev, b_ev, acc, 0, 0, 0);
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_od, b_od, acc, 0, 0, 0);
@@ -299,330 +282,492 @@ __global__ __launch_bounds__(256, 2) void k_q2g_gu_wk(
     }
 }
 
-template <int NCH, int MODE, bool SBL, int SBF>
-__global__ __launch_bounds__(256, 2) void k_q2g_proj(
+// ---- every K and any number of rows --------------------------------------------------------------
+//
+// Work.  A batch is up to TM M tiles of one segment (fewer where their activations would not fit in
+// LDS: 2 of 4 at K 2048 and 2560); an item is a batch times one column tile (WV waves, each one
+// (gate, up) pair of 16-row subtiles or two down subtiles: 16 intermediate or 32 output columns per
+// wave).  With span 0 a fixed grid (one block per CU at TM 4, two at TM 1) sums the items' costs
+// over the segments, and each block takes its own equal part of them in the order (segment, batch,
+// column tile), so neither a long segment nor the last round of blocks leaves CUs idle (777 tokens
+// over 100 experts of 1152 x 320: 132 -> 55 us, where one block used to take a 140-row segment in
+// five passes of dependent round trips).  With span > 0 a block is one segment and `span` column tiles.
+//
+// A block stages a batch's activations once, for the whole K (split into even / odd fragments), and
+// then runs its column tiles without a barrier: the queue of outstanding loads holds weights only, so
+// they can be requested one or two steps (512 inputs each) ahead.  With activations staged chunk by chunk, each
+// wait for a chunk's activations also waited for the weights requested before them (loads retire in
+// order), which held the requests in flight to one chunk: 16-36 KB per CU, 3 TB/s.
+//
+// What bounds it: the dequantisation (19 VALU operations per 16 weights and lane, about 83 cycles
+// against 33 of matrix unit per M tile).  Every weight is dequantised once per batch, so 64-row
+// batches where they fit.  512 tokens, top-10 of 512 experts at 2560 x 640 bf16: gate/up 161 us (524
+// MB, 3.3 TB/s; VALU issuing 56% of the time), down 102 us; 2048 tokens: 313 and 171 us.  Both and the
+// combine: 284 -> 244 us and 597 -> 435 us against the chunk-by-chunk kernel this replaced (32 rows per
+// pass).  Two subtile pairs per wave (256-column tiles, 2.5 of them at 640): 211 and 136 us; 12 waves
+// per block: 188 and 111; phase 0 of a half built under the half before: 157 and 106.
+constexpr int kMaxTiles = 4;                             // M tiles per batch, at most
+constexpr int kMmSubs = 2;                               // 16-row weight subtiles per wave
+constexpr int kCUs = 256;
+
+// The activations' LDS image of a batch: per step of 512 inputs and 16-row tile 16 KB, row m of 64
+// 16-byte units (half, even / odd codes, word), unit v of a row stored at v ^ m in its low 4 bits so
+// that the 16 rows read at one unit index start at 16 different slots of a 256-byte bank cycle.
+// Per block: all 160 KB of a CU; 80 KB for two blocks; 32 KB (K <= 1024) for four of 4 waves.
+template <int TM, int WV>
+constexpr int lds_units() { return TM > 1 ? 10240 : WV == 8 ? 5120 : 2048; }
+constexpr int kTileUnits = kMT * 64;
+
+typedef uint32_t u32_a2 __attribute__((aligned(2)));     // two adjacent fp16 / bf16 values
+
+// Cost of an item in the units of the shares: the weights' bytes and their dequantisation cost about
+// what the multiplication of four tiles does.
+constexpr uint32_t kItemCost = 4;
+
+// PAIR: K is a multiple of 512 (no group past the end).  TM: M tiles per batch, at most.  WV: waves.
+template <int MODE, int SBF, bool PAIR, int TM, int WV>
+__global__ __launch_bounds__(64 * WV, TM == 1 ? 4 : 2) void k_q2g_mm(
     const __half* __restrict__ src, int n_src_rows, const int32_t* __restrict__ row_map,
     const int32_t* __restrict__ row_out, int n_out_rows,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot, int n_seg, int n_rows,
-    Q2Experts E, int n_slots, int hidden, int inter, int tiles_per_seg, __half* __restrict__ out) {
-    constexpr int kMaxMT = max_mt<MODE>();
-    constexpr bool kPrefetch = MODE == kGateUp;        // a short K (down) gains nothing from it
-    const int K = MODE == kGateUp ? hidden : inter;              // contraction length
-    const int N = MODE == kGateUp ? inter : hidden;              // output rows per projection
-    const int kg = K / 64;
-    // Gate/up runs two passes over the (segment, slice) items: the first takes the segments that
-    // need more than one batch of M tiles, whose blocks run longest, so that they are dispatched
-    // first; the second takes the rest (each block of a pass that is not its own exits at once).
-    int work, pass = 0;
-    if constexpr (MODE == kGateUp) {
-        const int items = n_seg * tiles_per_seg;
-        pass = (int)blockIdx.x >= items ? 1 : 0;
-        work = xcd_order((int)blockIdx.x - pass * items, items);
-    } else {
-        work = xcd_order(blockIdx.x, gridDim.x);
-    }
-    const int seg = work / tiles_per_seg, tile = work % tiles_per_seg;
-    if (seg >= n_seg) return;
-    int r0 = seg_start[seg], r1 = seg_start[seg + 1];
-    r0 = r0 < 0 ? 0 : (r0 > n_rows ? n_rows : r0);
-    r1 = r1 < r0 ? r0 : (r1 > n_rows ? n_rows : r1);
-    const int slot = seg_slot ? seg_slot[seg] : seg;
-    if (r1 == r0 || slot < 0 || slot >= n_slots) return;
-    if constexpr (MODE == kGateUp) {
-        if ((pass == 0) != (r1 - r0 > kMT * kMaxMT)) return;
-    }
+    Q2Experts E, int n_slots, int K, int N, int tiles, int mtmax, int span, int vec_out, __half* __restrict__ out) {
+    constexpr int kCols = MODE == kGateUp ? 16 : 32;           // columns per wave
+    const int batch_rows = kMT * mtmax;
+    __shared__ uint4 a_lds[lds_units<TM, WV>()];
+    unsigned long long* wsum = reinterpret_cast<unsigned long long*>(a_lds);        // the shares' scratch
+    int(*bound)[6] = reinterpret_cast<int(*)[6]>(a_lds + 64);      // first / end item: segment, batch, tile; rows, slot
 
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n = lane & 15, kq = lane >> 4;
-    const size_t code_row = (size_t)K / 4, sb_row = (size_t)kg;   // bytes / (scale, bias) pairs per weight row
-
-    // Weight row of lane n in subtile s = base_s + n: a wave-uniform base per subtile plus one
-    // per-lane offset shared by all subtiles.
-    const uint8_t* codes[kSub];
-    const uint32_t* sbp[kSub];                 // SBF 0: (scale, bias) words of the subtile's rows
-    const uint16_t* scp[kSub];                 // SBF 1 / 2: scales and biases
-    const uint16_t* bip[kSub];
-    bool rv[kSub];
-    int col[kSub];
-#pragma unroll
-    for (int s = 0; s < kSub; ++s) {
-        int base, p;
-        if (MODE == kGateUp) {
-            base = tile * 128 + wv * 32 + (s >> 1) * 16;
-            p = (s & 1) ? 1 : 0;
-        } else {
-            base = tile * 256 + wv * 64 + s * 16;
-            p = 2;
-        }
-        col[s] = base + n;
-        // N is a multiple of 64, so a subtile is wholly in range or wholly out; one that is out
-        // reads the last in-range subtile (unconditional loads) and is never written
-        rv[s] = base < N;
-        if (base >= N) base = N - 16;
-        const Q2Proj& P = E.p[p];
-        codes[s] = P.w + (size_t)slot * P.w_stride + (size_t)base * code_row;
-        sbp[s] = reinterpret_cast<const uint32_t*>(P.s + (size_t)slot * P.s_stride) + (size_t)base * sb_row;
-        scp[s] = reinterpret_cast<const uint16_t*>(P.s + (size_t)slot * P.s_stride) + (size_t)base * sb_row;
-        bip[s] = reinterpret_cast<const uint16_t*>(P.b + (size_t)slot * P.b_stride) + (size_t)base * sb_row;
-    }
-    const uint32_t lane_code0 = (uint32_t)((size_t)n * code_row + (size_t)kq * 16);
-    const uint32_t lane_sb0 = (uint32_t)((size_t)n * sb_row + kq);
-
-    // Scale/bias words.  With SBL (gate/up, K a multiple of 256 and at least 512: rows of 4 k
-    // words, so every 16-byte piece below is aligned) each wave loads them four chunks at a time
-    // into its own LDS area, one 16-byte piece per lane and subtile: lane (n, q) loads groups
-    // 16 jj + 4 q .. + 3 of its row n (a piece past the row's end is moved back to its last 4
-    // groups), and chunk j = 4 jj + c reads group 4 j + kq from the piece of lane (n, c).  One
-    // such load touches as many cache lines as one of the per-chunk 4-byte loads it replaces,
-    // and there are four times fewer of them.  The pieces of block jj + 1 are loaded after chunk
-    // 4 jj is multiplied and written to LDS by the staging of chunk 4 jj + 1 (the compiler moves
-    // that write up to the loads, so they are waited for once per block); two buffers, so block
-    // jj + 1 lands while block jj is read.  Without SBL the words are loaded with the codes.
-    constexpr bool kSbLds = SBL;
-    static_assert(!SBL || NCH >= 2, "the LDS path needs K >= 512");
-    __shared__ uint32_t sb_lds[kSbLds ? 2 : 1][4][kSub][kSbLds ? 256 : 1];
-    const uint32_t lane_row_sb = (uint32_t)((size_t)n * sb_row);
-    auto sb_piece = [&](int jj, int q) {                       // first group of lane (., q)'s piece
-        const int g0 = 16 * jj + 4 * q;
-        return g0 + 4 <= kg ? g0 : kg - 4;
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    auto seg_range = [&](int seg, int& r0, int& r1, int& slot) {
+        r0 = seg_start[seg];
+        r1 = seg_start[seg + 1];
+        r0 = r0 < 0 ? 0 : (r0 > n_rows ? n_rows : r0);
+        r1 = r1 < r0 ? r0 : (r1 > n_rows ? n_rows : r1);
+        slot = seg_slot ? seg_slot[seg] : seg;
+        if (slot < 0 || slot >= n_slots) r1 = r0;
     };
-    // a block's pieces on their way to LDS, one named register set per subtile (as an array the
-    // compiler keeps them in memory: in LDS, or in scratch with a wait right after the loads)
-    uint4 sbn0, sbn1, sbn2, sbn3;
-    static_assert(kSub == 4, "one named piece per subtile");
-    auto sbn = [&](int s) -> uint4& { return s == 0 ? sbn0 : s == 1 ? sbn1 : s == 2 ? sbn2 : sbn3; };
-    auto fetch_sb = [&](int jj) {
-        const int gs = sb_piece(jj, kq);
+
+    int seg, batch, tile0, seg_e, batch_e, tile_e, r0, r1, slot;
+    int first = 0;                                             // where the next batch's tiles begin
+    if (TM == 1 && span) {
+        // one block per segment and `span` column tiles, which takes the segment's batches in turn
+        const int work = xcd_order(blockIdx.x, gridDim.x), per_seg = (tiles + span - 1) / span;
+        seg = seg_e = work / per_seg;
+        first = tile0 = work % per_seg * span;
+        batch = 0;
+        batch_e = 0x7FFFFFFF;
+        tile_e = 0;
+        seg_range(seg, r0, r1, slot);
+    } else {
+        // this block's share of the items, ordered by (segment, batch, column tile): those whose start
+        // in the running cost lies in [total * b / nb, total * (b + 1) / nb)
+        const int per = (n_seg + 64 * WV - 1) / (64 * WV), s0 = t * per;
+        const int s1 = s0 + per < n_seg ? s0 + per : n_seg;
+        auto cost = [&](int rows, uint32_t& full, uint32_t& rem) {
+            full = (uint32_t)rows / batch_rows;
+            rem = ((uint32_t)rows % batch_rows + kMT - 1) / kMT;
+            return (unsigned long long)tiles * (full * (kItemCost + (uint32_t)mtmax) + (rem ? kItemCost + rem : 0u));
+        };
+        unsigned long long sum = 0;
+        uint32_t full, rem;
+        r0 = r1 = slot = 0;                                    // the thread's only segment, where it has one
+        for (int s = s0; s < s1; ++s) {
+            seg_range(s, r0, r1, slot);
+            sum += cost(r1 - r0, full, rem);
+        }
+        unsigned long long inc = sum;
 #pragma unroll
-        for (int s = 0; s < kSub; ++s) {
-            if constexpr (SBF == 0) {
-                sbn(s) = *reinterpret_cast<const uint4*>(sbp[s] + lane_row_sb + gs);
-            } else {                           // 4 scales and 4 biases (8-byte aligned: kg % 4 == 0)
-                const uint2 sc = *reinterpret_cast<const uint2*>(scp[s] + lane_row_sb + gs);
-                const uint2 bi = *reinterpret_cast<const uint2*>(bip[s] + lane_row_sb + gs);
-                sbn(s) = make_uint4(sb_word<SBF>(sc.x & 0xFFFFu, bi.x & 0xFFFFu), sb_word<SBF>(sc.x >> 16, bi.x >> 16),
-                                    sb_word<SBF>(sc.y & 0xFFFFu, bi.y & 0xFFFFu), sb_word<SBF>(sc.y >> 16, bi.y >> 16));
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned long long o = __shfl_up(inc, d, 64);
+            if (lane >= d) inc += o;
+        }
+        if (lane == 63) wsum[wv] = inc;
+        if (t < 2) {
+            bound[t][0] = n_seg;
+            bound[t][1] = bound[t][2] = bound[t][3] = bound[t][4] = bound[t][5] = 0;
+        }
+        __syncthreads();
+        unsigned long long pre = inc - sum, total = 0;
+#pragma unroll
+        for (int w = 0; w < WV; ++w) {
+            if (w < wv) pre += wsum[w];
+            total += wsum[w];
+        }
+        // any function of b that does not fall, is 0 at 0 and total at nb gives every item one block
+        const int me = xcd_order(blockIdx.x, gridDim.x);
+        const double share = (double)total / (double)gridDim.x;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const unsigned long long at = me + e == (int)gridDim.x ? total : (unsigned long long)(share * (me + e));
+            if (at < pre || at >= pre + sum) continue;
+            unsigned long long p = pre;
+            for (int s = s0; s < s1; ++s) {
+                if (per > 1) seg_range(s, r0, r1, slot);
+                const unsigned long long c = cost(r1 - r0, full, rem);
+                if (at < p + c) {
+                    uint32_t b = 0, tl = 0;
+                    if (at > p) {
+                        const uint32_t d = (uint32_t)(at - p), fb = (uint32_t)tiles * (kItemCost + (uint32_t)mtmax);
+                        b = d / fb < full ? d / fb : full;
+                        const uint32_t ic = kItemCost + (b < full ? (uint32_t)mtmax : rem);
+                        tl = (d - b * fb + ic - 1) / ic;
+                    }
+                    bound[e][0] = s;
+                    bound[e][1] = (int)b;
+                    bound[e][2] = (int)tl;
+                    bound[e][3] = r0;
+                    bound[e][4] = r1;
+                    bound[e][5] = slot;
+                    break;
+                }
+                p += c;
             }
         }
-    };
-    auto put_sb = [&](int jj) {
-#pragma unroll
-        for (int s = 0; s < kSub; ++s) reinterpret_cast<uint4*>(&sb_lds[jj & 1][wv][s][0])[lane] = sbn(s);
-    };
+        __syncthreads();
+        seg = __builtin_amdgcn_readfirstlane(bound[0][0]);
+        batch = __builtin_amdgcn_readfirstlane(bound[0][1]);
+        tile0 = __builtin_amdgcn_readfirstlane(bound[0][2]);
+        r0 = __builtin_amdgcn_readfirstlane(bound[0][3]);
+        r1 = __builtin_amdgcn_readfirstlane(bound[0][4]);
+        slot = __builtin_amdgcn_readfirstlane(bound[0][5]);
+        seg_e = __builtin_amdgcn_readfirstlane(bound[1][0]);
+        batch_e = __builtin_amdgcn_readfirstlane(bound[1][1]);
+        tile_e = __builtin_amdgcn_readfirstlane(bound[1][2]);
+    }
 
-    // The segment's rows are taken in batches of up to kMaxMT M tiles (32 rows); within a batch
-    // every K chunk's weights are loaded and dequantised once and multiplied into every tile, so
-    // a long segment costs one pass over its weights per batch, not one per tile.
-    //
-    // Activation chunks are staged in LDS, shared by the 4 waves: per tile 16 rows x 32 units of
-    // 16 bytes (256 inputs), unit v of row m stored at m * 32 + (v ^ m) so that the 16 lanes
-    // reading one unit column hit distinct banks.  Each thread stages 2 units per tile.
-    __shared__ uint4 a_lds[kMaxMT][kMT * 32];
-    const int t = threadIdx.x;
-    const int sm0 = t >> 5, sm1 = sm0 + 8, sv = t & 31;       // the two units this thread stages
+    const int kg = K / 64, nst = (kg + 7) / 8;                 // steps of 8 groups (K 512) per column tile
+    // the last step of a K that is no multiple of 512: with at most 4 groups left it has one half
+    const bool one_half = !PAIR && (kg & 7) >= 1 && (kg & 7) <= 4;
+    const int n = lane & 15, kq = lane >> 4;
+    const uint32_t code_row = (uint32_t)K / 4;
+    // Weight row of lane n in subtile s: the wave's columns are dealt out so that a lane of the
+    // product (4 rows of the subtile) holds adjacent columns over all its subtiles
+    constexpr int kSubs = MODE == kGateUp ? 1 : 2;             // subtiles per projection
+    const uint32_t lane_row = (uint32_t)(4 * kSubs * (n >> 2) + (n & 3));
+    const uint32_t lane_code = lane_row * code_row, lane_sb = lane_row * (uint32_t)kg;
+    constexpr uint32_t kStep = SBF == 0 ? 4 : 2;
 
-    for (int b0 = r0; b0 < r1; b0 += kMT * kMaxMT) {
-        const int rows = (r1 - b0) < kMT * kMaxMT ? (r1 - b0) : kMT * kMaxMT;
-        const int mts = (rows + kMT - 1) / kMT;                // tiles in this batch (wave-uniform)
-        // The weight loads do not depend on the batch; an opaque copy of the lane offsets keeps
-        // the compiler from hoisting (and holding) a short K's whole weight slice across batches.
-        uint32_t lane_code = lane_code0, lane_sb = lane_sb0;
-        asm volatile("" : "+v"(lane_code), "+v"(lane_sb));
-        // source rows of the staged units; a row past the segment or naming an out-of-range
-        // source row is staged as zeros
-        int sr[kMaxMT][2];
+    // Group of lane group q in half h of step p: the two adjacent groups 2q, 2q + 1 of the step's
+    // eight, so a lane's codes are 32 contiguous bytes and its scales one word.  Groups past the
+    // end read the last one; their activations are staged as zeros.
+    auto group = [&](int p, int q, int h) {
+        if constexpr (PAIR) return 8 * p + 2 * q + h;
+        else return one_half && p == nst - 1 ? 8 * p + q : 8 * p + 2 * q + h;
+    };
+    auto clampg = [&](int g) { return PAIR ? g : (g < kg ? g : kg - 1); };
+    const int sv = t & 15;                                     // staged word: lane group sv >> 2, word sv & 3
+    constexpr int kPassRows = 4 * WV;                    // rows staged per pass of the block
+
+    // Rows b0 .. of one batch (M tiles, rows up to r1) times the column tiles ta .. tb - 1.
+    auto body = [&](auto mtc, int slot, int b0, int r1, int ta, int tb) {
+        constexpr int M = decltype(mtc)::value;
+        constexpr int U = (M * kMT + kPassRows - 1) / kPassRows;
+        const int sm = t >> 4;
+        const bool mine = M * kMT % kPassRows == 0 || (U - 1) * kPassRows + sm < M * kMT;   // last pass partial
+        const __half* xp[U];
 #pragma unroll
-        for (int mt = 0; mt < kMaxMT; ++mt) {
+        for (int u = 0; u < U; ++u) {
+            int r = b0 + u * kPassRows + sm;
+            r = r < r1 ? r : r1 - 1;
+            int v = row_map ? row_map[r] : r;
+            v = v >= 0 && v < n_src_rows ? v : 0;
+            xp[u] = src + (size_t)v * K + (sv & 3) * 16;
+        }
+        // the output row of this lane's row in each tile (-1: none), and for gate/up whether it names a
+        // source row (one that names none gives zeros)
+        int orow[M];
+        bool live[M];
+#pragma unroll
+        for (int mt = 0; mt < M; ++mt) {
+            const int r = b0 + mt * kMT + n, rc = r < r1 ? r : r1 - 1;
+            int o = rc;
+            live[mt] = true;
+            if constexpr (MODE == kGateUp) {
+                const int v = row_map ? row_map[rc] : rc;
+                live[mt] = v >= 0 && v < n_src_rows;
+            } else {
+                if (row_out) o = row_out[rc];
+                if (o >= n_out_rows) o = -1;
+            }
+            orow[mt] = r < r1 ? o : -1;
+        }
+        struct X {
+            uint4 v[U][2][2];
+        };
+        auto load_x = [&](int p, X& xs) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int m = mt * kMT + (h ? sm1 : sm0);
-                int v = -1;
-                if (m < rows) {
-                    const int r = b0 + m;
-                    v = row_map ? row_map[r] : r;
-                    if (v < 0 || v >= n_src_rows) v = -1;
-                }
-                sr[mt][h] = v;
-            }
-        }
-
-        f32x4 acc[kMaxMT][kSub];
+                const int g = clampg(group(p, sv >> 2, h));
 #pragma unroll
-        for (int mt = 0; mt < kMaxMT; ++mt)
-#pragma unroll
-            for (int s = 0; s < kSub; ++s) acc[mt][s] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-        uint4 cwa[kSub], cwb[kSub];                            // weights of the current / next chunk
-        uint32_t swa[kSub], swb[kSub];
-        uint4 xs[kMaxMT][2];                                   // staged activation units in flight
-        // Loads are unconditional from clamped in-range addresses and nothing masks them where
-        // they land: a load whose value is selected right away is sunk into a branch by the
-        // compiler, which then waits for it at the join and serialises a chunk's round trips.
-        // Groups past K (a K that is not a multiple of 256) read group kg - 1: their activations
-        // are staged as zeros, so those finite weights add nothing.  Rows past the segment and
-        // out-of-range source rows are zeroed when staged.
-        auto load_w = [&](int j, uint4 (&cw)[kSub], uint32_t (&sw)[kSub]) {
-            const bool gv = 4 * j + kq < kg;
-            const int gdelta = gv ? 0 : (kg - 1) - (4 * j + kq);      // clamp to group kg - 1
-#pragma unroll
-            for (int s = 0; s < kSub; ++s) {
-                cw[s] = *reinterpret_cast<const uint4*>(codes[s] + lane_code + (size_t)j * 64 + (ptrdiff_t)gdelta * 16);
-                if constexpr (!kSbLds) {
-                    const uint32_t gi = lane_sb + 4 * j + gdelta;
-                    if constexpr (SBF == 0) sw[s] = sbp[s][gi];
-                    else sw[s] = sb_word<SBF>(scp[s][gi], bip[s][gi]);
+                for (int u = 0; u < U; ++u) {
+                    const uint4* x = reinterpret_cast<const uint4*>(xp[u] + g * 64);
+                    xs.v[u][h][0] = x[0];
+                    xs.v[u][h][1] = x[1];
                 }
             }
         };
-        // After chunk j's multiply (j = 4 jj): the loads of the next block's words (needed from
-        // chunk 4 jj + 4 on); staging chunk j + 1 writes them to the buffer of block jj - 1, which
-        // the wave's reads have left.
-        auto next_sb_block = [&](int j) {
-            if constexpr (kSbLds) {
-                if ((j & 3) == 0 && 4 * ((j >> 2) + 1) < NCH) fetch_sb((j >> 2) + 1);
-            }
-        };
-        auto stage_sb = [&](int j) {
-            if constexpr (kSbLds) {
-                if (j == 0) put_sb(0);
-                else if ((j & 3) == 1 && 4 * ((j >> 2) + 1) < NCH) put_sb((j >> 2) + 1);
-            }
-        };
-        auto load_x = [&](int j) {
-            const int u = 32 * j + sv;                         // 16-byte unit within the row
-            const int uc = u * 8 < K ? u : K / 8 - 1;
+        auto stage = [&](int p, const X& xs) {
 #pragma unroll
-            for (int mt = 0; mt < kMaxMT; ++mt) {
-                if (mt >= mts) break;
+            for (int h = 0; h < 2; ++h) {
+                const bool uv = PAIR || group(p, sv >> 2, h) < kg;
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int v = sr[mt][h] < 0 ? 0 : sr[mt][h];
-                    xs[mt][h] = reinterpret_cast<const uint4*>(src + (size_t)v * K)[uc];
-                }
-            }
-        };
-        auto stage = [&](int j) {
-            const bool uv = (32 * j + sv) * 8 < K;
-#pragma unroll
-            for (int mt = 0; mt < kMaxMT; ++mt) {
-                if (mt >= mts) break;
-                a_lds[mt][sm0 * 32 + (sv ^ sm0)] = (sr[mt][0] >= 0 && uv) ? xs[mt][0] : make_uint4(0, 0, 0, 0);
-                a_lds[mt][sm1 * 32 + (sv ^ sm1)] = (sr[mt][1] >= 0 && uv) ? xs[mt][1] : make_uint4(0, 0, 0, 0);
-            }
-        };
-        // Per 32-bit word q of the lane's group: the activation fragments of every tile, then per
-        // subtile the two dequantised weight fragments, multiplied into every tile.
-        auto compute = [&](int j, const uint4 (&cw)[kSub], const uint32_t (&sw)[kSub]) {
-            uint32_t swv[kSub];
-#pragma unroll
-            for (int s = 0; s < kSub; ++s) swv[s] = sw[s];
-            if constexpr (kSbLds) {
-                const int c = j & 3, jj = j >> 2;
-                int e = 16 * jj + 4 * c + kq - sb_piece(jj, c);       // > 3 only for a group past K
-                e = e > 3 ? 3 : e;
-#pragma unroll
-                for (int s = 0; s < kSub; ++s) swv[s] = sb_lds[jj & 1][wv][s][(16 * c + n) * 4 + e];
-            }
-            f16x2 s2[kSub], b2[kSub];
-#pragma unroll
-            for (int s = 0; s < kSub; ++s) {
-                const f16x2 sb = __builtin_bit_cast(f16x2, swv[s]);
-                const _Float16 two_s = sb.x * (_Float16)2.0f;
-                s2[s] = (f16x2){two_s, two_s};
-                b2[s] = (f16x2){sb.y, sb.y};
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int v = 8 * kq + 2 * q;
-                f16x8 a_ev[kMaxMT], a_od[kMaxMT];
-#pragma unroll
-                for (int mt = 0; mt < kMaxMT; ++mt) {
-                    if (mt >= mts) break;
-                    const uint4* arow = a_lds[mt] + n * 32;
-                    split_even_odd(arow[v ^ n], arow[(v + 1) ^ n], a_ev[mt], a_od[mt]);
-                }
-#pragma unroll
-                for (int s = 0; s < kSub; ++s) {
-                    const uint32_t w = q == 0 ? cw[s].x : q == 1 ? cw[s].y : q == 2 ? cw[s].z : cw[s].w;
-                    const f16x8 b_ev = dequant8(w & 0x33333333u, s2[s], b2[s]);
-                    const f16x8 b_od = dequant8((w >> 2) & 0x33333333u, s2[s], b2[s]);
-#pragma unroll
-                    for (int mt = 0; mt < kMaxMT; ++mt) {
-                        if (mt >= mts) break;
-                        acc[mt][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_ev[mt], b_ev, acc[mt][s], 0, 0, 0);
-                        acc[mt][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_od[mt], b_od, acc[mt][s], 0, 0, 0);
+                for (int u = 0; u < U; ++u) {
+                    f16x8 ev, od;
+                    split_even_odd(xs.v[u][h][0], xs.v[u][h][1], ev, od);
+                    const int row = u * kPassRows + sm;
+                    uint4* d = a_lds + p * (M * kTileUnits) + row * 64 + 32 * h + (sv ^ (row & 15));
+                    if (u < U - 1 || mine) {
+                        d[0] = uv ? __builtin_bit_cast(uint4, ev) : make_uint4(0, 0, 0, 0);
+                        d[16] = uv ? __builtin_bit_cast(uint4, od) : make_uint4(0, 0, 0, 0);
                     }
                 }
             }
         };
-        // Software pipeline, one chunk deep: chunk j + 1's weights and activations are in flight
-        // while chunk j is multiplied (the activation registers are free once chunk j is staged).
-        // Loads retire in issue order: staging chunk j + 1 waits for its activations, and with
-        // them for chunk j + 1's weights, issued before them and needed next anyway.  The last
-        // chunk's look-ahead re-reads the last chunk (an L2 hit), so no load is conditional.
-        if constexpr (kSbLds) fetch_sb(0);
-        if constexpr (kPrefetch) {
-            load_x(0);
-            load_w(0, cwa, swa);
-#pragma unroll 1
-            for (int j = 0; j < NCH; ++j) {
-                load_w(j + 1 < NCH ? j + 1 : NCH - 1, cwb, swb);
-                lds_barrier();                                 // every wave is done with chunk j - 1
-                stage(j);
-                stage_sb(j);
-                lds_barrier();
-                load_x(j + 1 < NCH ? j + 1 : NCH - 1);
-                compute(j, cwa, swa);
-                next_sb_block(j);
+
+        // one step's weights: codes, and scale / bias words as loaded
+        struct W {
+            uint4 c[kMmSubs][2];
+            uint32_t r0[kMmSubs], r1[kMmSubs];
+        };
+        uint32_t sb[kMmSubs][2];
+        // Subtile s of column tile tl: 16 of the weight rows base .. of its projection.  N is a
+        // multiple of 64, so a wave's columns are wholly in range or wholly out; a wave that is out
+        // reads the last ones and does not write.
+        auto base_of = [&](int tl) { return (tl * WV + wv) * kCols; };
+        auto row_of = [&](int tl, int s) {
+            int base = base_of(tl);
+            base = base < N ? base : N - kCols;
+            return base + 4 * (MODE == kGateUp ? s >> 1 : s);
+        };
+        auto load_w = [&](int tl, int p, W& w) {
+            const uint32_t o0 = lane_code + (uint32_t)clampg(group(p, kq, 0)) * 16;
+            const uint32_t o1 = PAIR ? o0 + 16 : lane_code + (uint32_t)clampg(group(p, kq, 1)) * 16;
 #pragma unroll
-                for (int s = 0; s < kSub; ++s) {
-                    cwa[s] = cwb[s];
-                    swa[s] = swb[s];
+            for (int s = 0; s < kMmSubs; ++s) {
+                const Q2Proj& P = E.p[MODE == kGateUp ? (s & 1) : 2];
+                const uint8_t* c = P.w + (size_t)slot * P.w_stride + (size_t)row_of(tl, s) * code_row;
+                w.c[s][0] = *reinterpret_cast<const uint4*>(c + o0);
+                w.c[s][1] = *reinterpret_cast<const uint4*>(c + o1);
+            }
+        };
+        auto load_sb = [&](int tl, int p, W& w) {
+            const int g0 = clampg(group(p, kq, 0)), g1 = PAIR ? g0 + 1 : clampg(group(p, kq, 1));
+#pragma unroll
+            for (int s = 0; s < kMmSubs; ++s) {
+                const Q2Proj& P = E.p[MODE == kGateUp ? (s & 1) : 2];
+                const size_t ro = (size_t)row_of(tl, s) * (kg * kStep);
+                const uint8_t* sp = P.s + (size_t)slot * P.s_stride + ro;
+                const uint8_t* bp = P.b + (size_t)slot * P.b_stride + ro;
+                if constexpr (SBF == 0) {
+                    w.r0[s] = *reinterpret_cast<const uint32_t*>(sp + (lane_sb + (uint32_t)g0) * kStep);
+                    w.r1[s] = *reinterpret_cast<const uint32_t*>(sp + (lane_sb + (uint32_t)g1) * kStep);
+                } else if (PAIR || kg > 1) {
+                    // both groups with one load; from the last group of a row the one before it comes along
+                    const int gp = PAIR || g0 < kg - 1 ? g0 : kg - 2;
+                    const uint32_t o = (lane_sb + (uint32_t)gp) * kStep;
+                    w.r0[s] = *reinterpret_cast<const u32_a2*>(sp + o);
+                    w.r1[s] = *reinterpret_cast<const u32_a2*>(bp + o);
+                } else {
+                    w.r0[s] = *reinterpret_cast<const uint16_t*>(sp + lane_sb * kStep);
+                    w.r1[s] = *reinterpret_cast<const uint16_t*>(bp + lane_sb * kStep);
                 }
             }
-        } else {
-#pragma unroll 1
-            for (int j = 0; j < NCH; ++j) {
-                load_x(j);
-                load_w(j, cwa, swa);
-                lds_barrier();                                 // every wave is done with chunk j - 1
-                stage(j);
-                stage_sb(j);
-                lds_barrier();
-                compute(j, cwa, swa);
-                next_sb_block(j);
+        };
+        // of the step p that w holds
+        auto convert_sb = [&](int p, const W& w) {
+            const int drop = SBF == 0 || PAIR || kg == 1 || clampg(group(p, kq, 0)) < kg - 1 ? 0 : 16;
+#pragma unroll
+            for (int s = 0; s < kMmSubs; ++s) {
+                if constexpr (SBF == 0) {
+                    sb[s][0] = w.r0[s];
+                    sb[s][1] = w.r1[s];
+                } else {
+                    const uint32_t sc = PAIR ? w.r0[s] : w.r0[s] >> drop, bi = PAIR ? w.r1[s] : w.r1[s] >> drop;
+                    sb[s][0] = sb_word<SBF>(sc & 0xFFFFu, bi & 0xFFFFu);
+                    sb[s][1] = sb_word<SBF>(sc >> 16, bi >> 16);
+                }
             }
-        }
+        };
 
-        // Epilogue: lane holds rows 4*kq + i (i = 0..3) of column n of each subtile of each tile.
+        f32x4 acc[M][kMmSubs];
+        auto clear = [&]() {
 #pragma unroll
-        for (int mt = 0; mt < kMaxMT; ++mt) {
-            if (mt >= mts) break;
+            for (int mt = 0; mt < M; ++mt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = mt * kMT + 4 * kq + i;
-                if (m >= rows) continue;
-                const int r = b0 + m;
-                if (MODE == kGateUp) {
+                for (int s = 0; s < kMmSubs; ++s) acc[mt][s] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        };
+        // Eight phases per half (word q = ph / 2 of the lane's group, even or odd codes): a phase
+        // multiplies its fragments while the next phase's are read from LDS and dequantised, the two
+        // interleaved so that the matrix unit runs under the conversions.
+        const uint4* aq[4];
 #pragma unroll
-                    for (int p = 0; p < 2; ++p) {
-                        if (!rv[2 * p]) continue;
-                        const float g = acc[mt][2 * p][i], u = acc[mt][2 * p + 1][i];
-                        out[(size_t)r * N + col[2 * p]] = __float2half_rn(g / (1.0f + __expf(-g)) * u);
+        for (int q = 0; q < 4; ++q) aq[q] = a_lds + n * 64 + ((4 * kq + q) ^ n);
+        auto compute = [&](int p, const W& w, auto hc) {
+            constexpr int h = decltype(hc)::value;
+            const int po = p * (M * kTileUnits);
+            auto frag_a = [&](int ph, f16x8 (&a)[M]) {
+#pragma unroll
+                for (int mt = 0; mt < M; ++mt)
+                    a[mt] = __builtin_bit_cast(f16x8, aq[ph >> 1][po + mt * kTileUnits + 32 * h + 16 * (ph & 1)]);
+            };
+            auto frag_b = [&](int ph, f16x8 (&b)[kMmSubs]) {
+#pragma unroll
+                for (int s = 0; s < kMmSubs; ++s) {
+                    const int q = ph >> 1;
+                    const uint4 cv = w.c[s][h];
+                    const uint32_t wq = q == 0 ? cv.x : q == 1 ? cv.y : q == 2 ? cv.z : cv.w;
+                    b[s] = dequant8((wq >> (2 * (ph & 1))) & 0x33333333u, sb[s][h]);
+                }
+            };
+            f16x8 fa[2][M], fb[2][kMmSubs];
+            frag_a(0, fa[0]);
+            frag_b(0, fb[0]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ph = 0; ph < 8; ++ph) {
+                if (ph < 7) {
+                    frag_a(ph + 1, fa[(ph + 1) & 1]);
+                    frag_b(ph + 1, fb[(ph + 1) & 1]);
+                }
+#pragma unroll
+                for (int s = 0; s < kMmSubs; ++s)
+#pragma unroll
+                    for (int mt = 0; mt < M; ++mt)
+                        acc[mt][s] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[ph & 1][s], fa[ph & 1][mt], acc[mt][s], 0, 0, 0);
+                if (ph < 7) {
+                    constexpr int kPer = (10 * kMmSubs + kMmSubs * M - 1) / (kMmSubs * M);
+                    __builtin_amdgcn_sched_group_barrier(0x100, M, 0);
+#pragma unroll
+                    for (int i = 0; i < kMmSubs * M; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, kPer, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        // lane: row n of each tile, 4 * kSubs adjacent columns
+        auto write = [&](int tl) {
+            if (base_of(tl) >= N) return;
+#pragma unroll
+            for (int mt = 0; mt < M; ++mt) {
+                if (orow[mt] < 0) continue;
+                __half* o = out + (size_t)orow[mt] * N + base_of(tl) + 4 * kSubs * kq;
+                uint32_t hw[2 * kSubs];
+#pragma unroll
+                for (int i = 0; i < 2 * kSubs; ++i) {
+                    uint32_t v[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const int c = 2 * i + e, s = c >> 2;
+                        if constexpr (MODE == kGateUp) {
+                            const float g = acc[mt][2 * s][c & 3], u = acc[mt][2 * s + 1][c & 3];
+                            v[e] = __half_as_ushort(__float2half_rn(live[mt] ? g / (1.0f + __expf(-g)) * u : 0.0f));
+                        } else {
+                            v[e] = __half_as_ushort(__float2half_rn(acc[mt][s][c & 3]));
+                        }
+                    }
+                    hw[i] = v[0] | (v[1] << 16);
+                }
+                if (vec_out) {
+                    if constexpr (kSubs == 1) {
+                        *reinterpret_cast<uint2*>(o) = make_uint2(hw[0], hw[1]);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < kSubs / 2; ++i)
+                            reinterpret_cast<uint4*>(o)[i] =
+                                make_uint4(hw[4 * i], hw[4 * i + 1], hw[4 * i + 2], hw[4 * i + 3]);
                     }
                 } else {
-                    const int orow = row_out ? row_out[r] : r;
-                    if (orow < 0 || orow >= n_out_rows) continue;
 #pragma unroll
-                    for (int s = 0; s < kSub; ++s)
-                        if (rv[s]) out[(size_t)orow * N + col[s]] = __float2half_rn(acc[mt][s][i]);
+                    for (int i = 0; i < 4 * kSubs; ++i)
+                        o[i] = __ushort_as_half((unsigned short)(hw[i >> 1] >> (16 * (i & 1))));
                 }
             }
+        };
+
+        // The batch's activations are staged once for the whole K; after that the waves run without
+        // barriers.  One step = 512 inputs of one column tile: its weights are loaded two steps ahead
+        // (past the end the last step's are read again: no load is conditional).
+        int tl = ta, p = 0, tl_w = ta, p_w = 0;
+        // steps ahead; one at four waves per SIMD, whose 128 registers do not hold a third step (spills:
+        // 2560 x 640, 37 tokens 134 us against 121)
+        constexpr int kAhead = TM == 1 ? 1 : 2;
+        W w0, w1, w2;
+        auto fetch = [&](W& w) {
+            load_w(tl_w, p_w, w);
+            load_sb(tl_w, p_w, w);
+            if (p_w + 1 < nst) {
+                ++p_w;
+            } else if (tl_w + 1 < tb) {
+                ++tl_w;
+                p_w = 0;
+            }
+        };
+        {
+            X xa, xb;
+            load_x(0, xa);
+            load_x(nst > 1 ? 1 : 0, xb);
+            fetch(w0);
+            if constexpr (kAhead == 2) fetch(w1);
+            lds_barrier();                                     // every wave is done with the LDS
+            stage(0, xa);
+            if (nst > 1) stage(1, xb);
+            for (int q = 2; q < nst; q += 2) {
+                load_x(q, xa);
+                load_x(q + 1 < nst ? q + 1 : q, xb);
+                stage(q, xa);
+                if (q + 1 < nst) stage(q + 1, xb);
+            }
+            lds_barrier();
         }
-        __syncthreads();                                       // a_lds is reused by the next batch
+        clear();
+        auto step = [&](const W& cur, W& nxt) {
+            fetch(nxt);
+            __builtin_amdgcn_sched_barrier(0);
+            convert_sb(p, cur);
+            compute(p, cur, std::integral_constant<int, 0>());
+            if (PAIR || !(one_half && p == nst - 1)) compute(p, cur, std::integral_constant<int, 1>());
+            if (++p < nst) return true;
+            write(tl);
+            clear();
+            p = 0;
+            return ++tl < tb;
+        };
+        for (;;) {
+            if constexpr (kAhead == 2) {
+                if (!step(w0, w2)) break;
+                if (!step(w1, w0)) break;
+                if (!step(w2, w1)) break;
+            } else {
+                if (!step(w0, w1)) break;
+                if (!step(w1, w0)) break;
+            }
+        }
+    };
+
+    while (seg < n_seg && (seg < seg_e || (seg == seg_e && batch <= batch_e))) {
+        const int b0 = r0 + batch * batch_rows;
+        if (b0 >= r1) {
+            batch = tile0 = 0;
+            if (++seg < n_seg && seg <= seg_e) seg_range(seg, r0, r1, slot);
+            continue;
+        }
+        const bool at_end = seg == seg_e && batch == batch_e;
+        const int tb = TM == 1 && span ? (first + span < tiles ? first + span : tiles) : at_end ? tile_e : tiles;
+        if (tile0 < tb) {
+            const int mts = (r1 - b0 + kMT - 1) / kMT;
+            if (TM == 1 || mtmax == 1 || mts == 1) body(std::integral_constant<int, 1>(), slot, b0, r1, tile0, tb);
+            else if (mtmax == 2 || mts == 2) body(std::integral_constant<int, TM == 1 ? 1 : 2>(), slot, b0, r1, tile0, tb);
+            else if (mtmax == 3 || mts == 3) body(std::integral_constant<int, TM == 1 ? 1 : 3>(), slot, b0, r1, tile0, tb);
+            else body(std::integral_constant<int, TM>(), slot, b0, r1, tile0, tb);
+        }
+        if (at_end) break;
+        ++batch;
+        tile0 = first;
     }
 }
-
 
 // Down in the whole-K form (K = inter = 256 * GPL): a block takes one segment and 256 output rows,
 // each wave 4 subtiles of 16 rows whose whole K it requests at once and keeps in registers while
@@ -725,14 +870,9 @@ __global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
         const uint4* arow = a_lds + n * UPR;
 #pragma unroll
         for (int i = 0; i < GPL; ++i) {
-            f16x2 s2[4], b2[4];
+            uint32_t sb[4];
 #pragma unroll
-            for (int sIdx = 0; sIdx < 4; ++sIdx) {
-                const f16x2 sb = __builtin_bit_cast(f16x2, sw[sIdx][i] ^ z);
-                const _Float16 two_s = sb.x * (_Float16)2.0f;
-                s2[sIdx] = (f16x2){two_s, two_s};
-                b2[sIdx] = (f16x2){sb.y, sb.y};
-            }
+            for (int sIdx = 0; sIdx < 4; ++sIdx) sb[sIdx] = sw[sIdx][i] ^ z;
             const int u0 = 8 * (GPL * kq + i);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -743,8 +883,8 @@ __global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
                 for (int sIdx = 0; sIdx < 4; ++sIdx) {
                     const uint4 cv = cw[sIdx][i];
                     const uint32_t wq = (q == 0 ? cv.x : q == 1 ? cv.y : q == 2 ? cv.z : cv.w) ^ z;
-                    const f16x8 b_ev = dequant8(wq & 0x33333333u, s2[sIdx], b2[sIdx]);
-                    const f16x8 b_od = dequant8((wq >> 2) & 0x33333333u, s2[sIdx], b2[sIdx]);
+                    const f16x8 b_ev = dequant8(wq & 0x33333333u, sb[sIdx]);
+                    const f16x8 b_od = dequant8((wq >> 2) & 0x33333333u, sb[sIdx]);
                     acc[sIdx] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_ev, b_ev, acc[sIdx], 0, 0, 0);
                     acc[sIdx] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_od, b_od, acc[sIdx], 0, 0, 0);
                 }
@@ -765,31 +905,52 @@ __global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
     }
 }
 
-template <int NCH, int MODE, bool SBL, int SBF>
-int launch_proj(const __half* src, int n_src_rows, const int32_t* row_map, const int32_t* row_out, int n_out_rows,
-                const int32_t* seg_start, const int32_t* seg_slot, int n_seg, int n_rows, const Q2Experts& E,
-                int n_slots, int hidden, int inter, __half* out, hipStream_t s) {
-    const int N = MODE == kGateUp ? inter : hidden;
-    const int rows_per_block = MODE == kGateUp ? 128 : 256;
-    const int tiles = (N + rows_per_block - 1) / rows_per_block;
-    // K = 512 exactly (whole 256-wide chunks): down in the whole-K form
-    const bool dn_wk = MODE == kDown && NCH == 2 && !SBL && inter == 256 * NCH;
-    const long long nb = (MODE == kGateUp || dn_wk ? 2LL : 1LL) * n_seg * tiles;   // two passes
-    if (nb <= 0) return 0;
+template <int MODE, int SBF, int TM, int WV>
+int launch_mm(int K, int span, const __half* src, int n_src_rows, const int32_t* row_map, const int32_t* row_out,
+              int n_out_rows, const int32_t* seg_start, const int32_t* seg_slot, int n_seg, int n_rows,
+              const Q2Experts& E, int n_slots, int N, __half* out, hipStream_t s) {
+    constexpr int cols = WV * (MODE == kGateUp ? 16 : 32), cus = TM == 1 ? 2 * kCUs : kCUs;
+    const int tiles = (N + cols - 1) / cols, nst = (K + 511) / 512;
+    const int fit = lds_units<TM, WV>() / (nst * kTileUnits), mtmax = fit < TM ? fit : TM;
+    const long long items = (long long)tiles * (n_seg + (long long)n_rows / (kMT * mtmax));   // at most
+    const long long nbl = span ? (long long)n_seg * ((tiles + span - 1) / span) : items < cus ? items : cus;
+    if (nbl > 0x7FFFFFFFLL) { moe_set_error("grouped q2: grid too large"); return -1; }
+    const unsigned nb = (unsigned)nbl;
+    const int vec_out = (uintptr_t)out % 16 == 0;              // rows are whole 128-byte lines; the base may not be
+    if (K % 512 == 0)
+        MOE_LAUNCH(MODE == kGateUp ? TK_PF_GATE_UP : TK_PF_DOWN, (k_q2g_mm<MODE, SBF, true, TM, WV>), dim3(nb),
+                   dim3(64 * WV), 0, s, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg,
+                   n_rows, E, n_slots, K, N, tiles, mtmax, span, vec_out, out);
+    else
+        MOE_LAUNCH(MODE == kGateUp ? TK_PF_GATE_UP : TK_PF_DOWN, (k_q2g_mm<MODE, SBF, false, TM, WV>), dim3(nb),
+                   dim3(64 * WV), 0, s, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg,
+                   n_rows, E, n_slots, K, N, tiles, mtmax, span, vec_out, out);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+template <int SBF>
+int launch_gu_wk(const __half* src, int n_src_rows, const int32_t* row_map, const int32_t* seg_start,
+                 const int32_t* seg_slot, int n_seg, int n_rows, const Q2Experts& E, int n_slots, int inter,
+                 __half* out, hipStream_t s) {
+    const int tiles = (inter + 127) / 128;
+    const long long nb = 2LL * n_seg * tiles;                  // two passes
     if (nb > 0x7FFFFFFFLL) { moe_set_error("grouped q2: grid too large"); return -1; }
-    if (dn_wk) {
-        if constexpr (MODE == kDown && NCH == 2 && !SBL)
-            MOE_LAUNCH(TK_PF_DOWN, (k_q2g_dn_wk<NCH, SBF>), dim3((unsigned)nb), dim3(256), 0, s, src, n_src_rows, row_out,
-                       n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots, hidden, tiles, out);
-    } else if constexpr (MODE == kGateUp && SBL && NCH == 8) {
-        // K = 2048: the whole-K form (128 rows per block, as here)
-        MOE_LAUNCH(TK_PF_GATE_UP, (k_q2g_gu_wk<NCH, SBF>), dim3((unsigned)nb), dim3(256), 0, s, src, n_src_rows, row_map,
-                   seg_start, seg_slot, n_seg, n_rows, E, n_slots, inter, tiles, out);
-    } else {
-        MOE_LAUNCH(MODE == kGateUp ? TK_PF_GATE_UP : TK_PF_DOWN, (k_q2g_proj<NCH, MODE, SBL, SBF>), dim3((unsigned)nb),
-                   dim3(256), 0, s, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg, n_rows,
-                   E, n_slots, hidden, inter, tiles, out);
-    }
+    MOE_LAUNCH(TK_PF_GATE_UP, (k_q2g_gu_wk<8, SBF>), dim3((unsigned)nb), dim3(256), 0, s, src, n_src_rows, row_map,
+               seg_start, seg_slot, n_seg, n_rows, E, n_slots, inter, tiles, out);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+template <int SBF>
+int launch_dn_wk(const __half* src, int n_src_rows, const int32_t* row_out, int n_out_rows, const int32_t* seg_start,
+                 const int32_t* seg_slot, int n_seg, int n_rows, const Q2Experts& E, int n_slots, int hidden,
+                 __half* out, hipStream_t s) {
+    const int tiles = (hidden + 255) / 256;
+    const long long nb = 2LL * n_seg * tiles;                  // two passes
+    if (nb > 0x7FFFFFFFLL) { moe_set_error("grouped q2: grid too large"); return -1; }
+    MOE_LAUNCH(TK_PF_DOWN, (k_q2g_dn_wk<2, SBF>), dim3((unsigned)nb), dim3(256), 0, s, src, n_src_rows, row_out,
+               n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots, hidden, tiles, out);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -798,23 +959,52 @@ template <int MODE, int SBF>
 int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row_map, const int32_t* row_out,
                     int n_out_rows, const int32_t* seg_start, const int32_t* seg_slot, int n_seg, int n_rows,
                     const Q2Experts& E, int n_slots, int hidden, int inter, __half* out, hipStream_t s) {
-    // the four-chunk scale/bias blocks pay on gate/up's long K; down (K = inter, often 2 chunks)
-    // is faster with the per-chunk loads
-    const bool sbl = MODE == kGateUp && K % 256 == 0 && K >= 512;
-    switch ((K + 255) / 256) {
-#define PF_CASE(c) \
-    case c: \
-        if (sbl) \
-            return launch_proj<c, MODE, (c >= 2 && MODE == kGateUp), SBF>(src, n_src_rows, row_map, row_out, n_out_rows, \
-                                                                          seg_start, seg_slot, n_seg, n_rows, E, n_slots, \
-                                                                          hidden, inter, out, s); \
-        return launch_proj<c, MODE, false, SBF>(src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, \
-                                                n_seg, n_rows, E, n_slots, hidden, inter, out, s);
-        PF_CASE(1) PF_CASE(2) PF_CASE(3) PF_CASE(4) PF_CASE(5)
-        PF_CASE(6) PF_CASE(7) PF_CASE(8) PF_CASE(9) PF_CASE(10)
-#undef PF_CASE
-        default: moe_set_error("grouped q2: contraction length %d unsupported (<= %d)", K, kMaxChunks * 256); return -1;
+    // Few rows per expert at the two shapes the whole-K kernels are built for: those, whose short
+    // blocks (512 or more, 2-4 per CU) hide each other's latencies; from about one full M tile per
+    // expert on, k_q2g_mm's one pass over the weights per 64 rows wins (gate/up + down + combine, 512
+    // experts of 2048 x 512: 16 tokens x top-10 40 us against 58, 128 tokens 115 against 145, 512
+    // tokens 186 against 191, 2048 tokens 540 against 350).  The line is drawn on the pool's slots,
+    // not on the segments, so cutting segments into pieces does not change the kernel (nor a bit of
+    // the result).
+    if (n_rows < 16LL * n_slots) {
+        if constexpr (MODE == kGateUp) {
+            if (K == 2048)
+                return launch_gu_wk<SBF>(src, n_src_rows, row_map, seg_start, seg_slot, n_seg, n_rows, E, n_slots, inter,
+                                         out, s);
+        } else if (K == 512) {
+            return launch_dn_wk<SBF>(src, n_src_rows, row_out, n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots,
+                                     hidden, out, s);
+        }
     }
+    auto go = [&](auto tm, auto wv, int span) {
+        return launch_mm<MODE, SBF, decltype(tm)::value, decltype(wv)::value>(
+            K, span, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots,
+            MODE == kGateUp ? inter : hidden, out, s);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Four = std::integral_constant<int, 4>;
+    using Eight = std::integral_constant<int, 8>;
+    const int N = MODE == kGateUp ? inter : hidden;
+    // Short calls: blocks of one segment and a few column tiles instead of shares, so that no block starts
+    // with the sum over the segments (2-3 us), while the blocks are few and the segments short; K up
+    // to 1024 in blocks of 4 waves, four per CU.  Gate/up + down + combine in us (chunked kernel
+    // before; shares; these): 12 tokens x top-7 of 28 experts, 512 x 256: 13.8, 19.2, 11.7; 251 x
+    // top-4 of 381, 576 x 512: 45.5, 44.9, 40.4; 5 x top-7, 2176 x 576: 36.8, 33.7, 29.5.  The lines
+    // lie where the shares win again: 415 x top-6 of 289, 960 x 512 (8.6 rows per expert) 61.3
+    // against 63.4; 54 x top-8 of 95, 1216 x 448 (4.5 rows) 34.0 against 39.3; 64 x top-10 of 512,
+    // 2560 x 640 (367 segments, 1,835 blocks) 152 against 175.
+    const long long t4 = (N + (MODE == kGateUp ? 63 : 127)) / (MODE == kGateUp ? 64 : 128), t8 = (t4 + 1) / 2;
+    // A block takes as many column tiles as keep the grid at 2,048 blocks, 1,024 with the shortest
+    // segments (55 x top-3 of 401, 2240 x 256: 36.6 against 34.0; 415 x top-6 of 289: 65.7 against 75.3).
+    const long long most = n_rows <= 4LL * n_seg ? 1024 : 2048;
+    if (K <= 1024 && n_rows <= (n_rows <= 1024 ? 16LL : 10LL) * n_seg && n_seg * t4 <= 6144)
+        return go(One(), Four(), (int)((n_seg * t4 + most - 1) / most));
+    if (K > 1024 && n_rows <= 4LL * n_seg && n_seg * t8 <= 1024) return go(One(), Eight(), 1);
+    // One-tile batches, two blocks per CU, for few rows per segment (256 tokens at 2560 x 640, 5 per
+    // expert: 242 / 230 us against 246 / 232 with 64-row batches; 512 tokens, 10 per expert: 297 /
+    // 286 against 296 / 275) and for small work (1,660 x top-2 of 28, 256 x 512: 27.0 against 35.1).
+    if (n_rows <= 8LL * n_seg || (K <= 512 && n_rows <= 4096)) return go(One(), Eight(), 0);
+    return go(std::integral_constant<int, kMaxTiles>(), Eight(), 0);
 }
 
 template <int MODE>
