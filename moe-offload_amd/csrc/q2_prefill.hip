@@ -102,20 +102,45 @@ __device__ __forceinline__ uint32_t sb_word(uint32_t sc, uint32_t bi) {
     return (sc & 0xFFFFu) | (bi << 16);
 }
 
+// Four words of each of a wave's four 16-lane groups, transposed between the groups: afterwards
+// word p of group q is what word q of group p was.
+__device__ __forceinline__ void transpose4(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+    auto swap32 = [](uint32_t& x, uint32_t& y) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        x = r[0];
+        y = r[1];
+    };
+    auto swap16 = [](uint32_t& x, uint32_t& y) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        x = r[0];
+        y = r[1];
+    };
+    swap32(a, c);
+    swap32(b, d);
+    swap16(a, b);
+    swap16(c, d);
+}
+
 // Gate/up of one M tile (at most 16 rows r0 .. r0 + rows - 1 of a segment) and one 128-row slice,
 // the weight rows streamed whole: each wave owns two (gate, up) pairs of 16-row subtiles and
-// requests a pair's whole K at once (lane (n, kq) loads groups GPL*kq .. GPL*kq + GPL - 1 of row
-// n: 16 rows x 64 * GPL contiguous bytes per subtile), the second pair's loads issued before the
+// requests a pair's whole K at once (lane (n, kq) loads groups 8p + 2kq and 8p + 2kq + 1, p < 4, of
+// row n: 16 rows x 64 * GPL contiguous bytes per subtile), the second pair's loads issued before the
 // first pair is multiplied.  The tile's activation rows are staged in LDS once for the whole K,
 // already split into the MFMA's even / odd input fragments: one barrier per tile, after which the
-// waves run independently.  A K position of an MFMA pairs lane group kq's group GPL*kq + i with
+// waves run independently.  A K position of an MFMA pairs lane group kq's group 8p + 2kq + h with
 // the same inputs on the A side; the even/odd code split inside a word is the one described above.
-// Bit for bit this is not k_q2g_mm's sum order (another K order inside the MFMAs).
+// These are k_q2g_mm's positions in k_q2g_mm's order, so a row's h has the same bits whichever of
+// the two kernels a call's size selects.  (The other way round, a quarter of K per lane group in
+// both, costs k_q2g_mm 25% at this K: each of its steps would touch every line of a weight row.)
+// The 9-tensor form's scales and biases still come in one 16-byte load each, a quarter of a row per
+// lane group, and are dealt out between the groups in registers: 512 tokens, top-10 of 512, 2048 x
+// 512 bf16: 178 us for gate/up + down + combine, 190 with a 4-byte load per pair of groups.
 template <int GPL, int SBF>
 __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n_src_rows,
                                            const int32_t* __restrict__ row_map, int r0, int rows, int slot,
                                            int tile, const Q2Experts& E, int inter, __half* __restrict__ out,
                                            uint4* __restrict__ a_lds) {
+    static_assert(GPL == 8, "four steps of 8 groups");
     constexpr int K = 256 * GPL;
     constexpr int kg = 4 * GPL;                       // groups per weight row
     constexpr int UPR = K / 8;                        // 16-byte units per activation row
@@ -156,47 +181,51 @@ __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const Q2Proj& P = h ? Pu : Pg;
-            const uint8_t* cr = P.w + (size_t)slot * P.w_stride + (size_t)(base + n) * code_row + (size_t)(GPL * kq) * 16;
+            const uint8_t* cr = P.w + (size_t)slot * P.w_stride + (size_t)(base + n) * code_row + (size_t)kq * 32;
 #pragma unroll
-            for (int i = 0; i < GPL; ++i) c[h][i] = *reinterpret_cast<const uint4*>(cr + (size_t)i * 16);
+            for (int i = 0; i < GPL; ++i) c[h][i] = *reinterpret_cast<const uint4*>(cr + (i >> 1) * 128 + (i & 1) * 16);
             if constexpr (SBF == 0) {
-                static_assert(GPL % 4 == 0, "whole 16-byte scale/bias pieces");
                 const uint32_t* sr = reinterpret_cast<const uint32_t*>(P.s + (size_t)slot * P.s_stride) +
-                                     (size_t)(base + n) * kg + GPL * kq;
+                                     (size_t)(base + n) * kg + 2 * kq;
 #pragma unroll
-                for (int i = 0; i < GPL / 4; ++i) {
-                    const uint4 v = reinterpret_cast<const uint4*>(sr)[i];
-                    wd[h][4 * i] = v.x;
-                    wd[h][4 * i + 1] = v.y;
-                    wd[h][4 * i + 2] = v.z;
-                    wd[h][4 * i + 3] = v.w;
+                for (int i = 0; i < GPL; i += 2) {
+                    const uint2 v = *reinterpret_cast<const uint2*>(sr + 4 * i);
+                    wd[h][i] = v.x;
+                    wd[h][i + 1] = v.y;
                 }
             } else {
-                static_assert(GPL % 8 == 0, "whole 16-byte scale / bias pieces");
-                const uint16_t* scr = reinterpret_cast<const uint16_t*>(P.s + (size_t)slot * P.s_stride) +
-                                      (size_t)(base + n) * kg + GPL * kq;
-                const uint16_t* bir = reinterpret_cast<const uint16_t*>(P.b + (size_t)slot * P.b_stride) +
-                                      (size_t)(base + n) * kg + GPL * kq;
-#pragma unroll
-                for (int i = 0; i < GPL / 8; ++i) {
-                    const uint4 sc = reinterpret_cast<const uint4*>(scr)[i];
-                    const uint4 bi = reinterpret_cast<const uint4*>(bir)[i];
-                    const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w}, biw[4] = {bi.x, bi.y, bi.z, bi.w};
-#pragma unroll
-                    for (int k2 = 0; k2 < 4; ++k2) {
-                        wd[h][8 * i + 2 * k2] = sb_word<SBF>(scw[k2] & 0xFFFFu, biw[k2] & 0xFFFFu);
-                        wd[h][8 * i + 2 * k2 + 1] = sb_word<SBF>(scw[k2] >> 16, biw[k2] >> 16);
-                    }
-                }
+                // groups 8kq .. 8kq + 7, two to a word: scales in the even elements, biases in the odd
+                const size_t o = (size_t)(base + n) * (2 * kg) + 16 * kq;
+                const uint4 sc = *reinterpret_cast<const uint4*>(P.s + (size_t)slot * P.s_stride + o);
+                const uint4 bi = *reinterpret_cast<const uint4*>(P.b + (size_t)slot * P.b_stride + o);
+                wd[h][0] = sc.x, wd[h][2] = sc.y, wd[h][4] = sc.z, wd[h][6] = sc.w;
+                wd[h][1] = bi.x, wd[h][3] = bi.y, wd[h][5] = bi.z, wd[h][7] = bi.w;
             }
         }
     };
     auto multiply = [&](int pp, const uint4 (&c)[2][GPL], const uint32_t (&wd)[2][GPL]) {
         f32x4 accg = (f32x4){0.f, 0.f, 0.f, 0.f}, accu = (f32x4){0.f, 0.f, 0.f, 0.f};
         const uint4* arow = a_lds + n * UPR;
+        uint32_t w[2][GPL];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < GPL; ++i) w[h][i] = wd[h][i];
+            if constexpr (SBF != 0) {
+                transpose4(w[h][0], w[h][2], w[h][4], w[h][6]);
+                transpose4(w[h][1], w[h][3], w[h][5], w[h][7]);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < GPL; ++i) {
-            const int u0 = 8 * (GPL * kq + i);
+            const int u0 = 8 * (8 * (i >> 1) + 2 * kq + (i & 1));
+            uint32_t sb[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t sc = w[h][i & ~1], bi = w[h][i | 1];
+                if constexpr (SBF == 0) sb[h] = w[h][i];
+                else sb[h] = i & 1 ? sb_word<SBF>(sc >> 16, bi >> 16) : sb_word<SBF>(sc & 0xFFFFu, bi & 0xFFFFu);
+            }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int v = u0 + 2 * q;
@@ -206,8 +235,8 @@ __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n
                 for (int h = 0; h < 2; ++h) {
                     const uint4 cv = c[h][i];
                     const uint32_t wq = q == 0 ? cv.x : q == 1 ? cv.y : q == 2 ? cv.z : cv.w;
-                    const f16x8 b_ev = dequant8(wq & 0x33333333u, wd[h][i]);
-                    const f16x8 b_od = dequant8((wq >> 2) & 0x33333333u, wd[h][i]);
+                    const f16x8 b_ev = dequant8(wq & 0x33333333u, sb[h]);
+                    const f16x8 b_od = dequant8((wq >> 2) & 0x33333333u, sb[h]);
                     f32x4& acc = h ? accu : accg;
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_ev, b_ev, acc, 0, 0, 0);
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_od, b_od, acc, 0, 0, 0);
@@ -772,7 +801,8 @@ __global__ __launch_bounds__(64 * WV, TM == 1 ? 4 : 2) void k_q2g_mm(
 // Down in the whole-K form (K = inter = 256 * GPL): a block takes one segment and 256 output rows,
 // each wave 4 subtiles of 16 rows whose whole K it requests at once and keeps in registers while
 // the segment's 16-row tiles of h pass through LDS (staged for the whole K, split into the MFMA's
-// even / odd fragments; one barrier per tile).  Output row r goes to row_out[r] (or r).
+// even / odd fragments; one barrier per tile).  Output row r goes to row_out[r] (or r).  Lane group kq
+// takes groups 2kq and 2kq + 1: at K = 512 these are k_q2g_mm's positions, and the sums have its bits.
 template <int GPL, int SBF>
 __global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
     const __half* __restrict__ src, int n_src_rows, const int32_t* __restrict__ row_out, int n_out_rows,

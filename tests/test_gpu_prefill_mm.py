@@ -6,6 +6,7 @@ error of at most 2^-11 each, so the 2-norm of a segment's error is within 3 * 2^
   halves, whole steps, and the longest (2560); segments of 0, 1, 16, 17, 64, 65 and 130 rows; blob
   pools and the 9-tensor form with fp16 and bf16 scales; output columns below and above one tile;
 * more segments than threads in a block, over a pool of few slots, with long and empty ones mixed in;
+* the same rows in calls of different sizes, which select different kernels, give the same bits;
 * an output that starts 2 bytes past a 16-byte boundary, and rows that name no source row, no output
   row and no slot, are handled as by the other kernels.
 """
@@ -115,3 +116,42 @@ def test_mm_out_of_range_and_unaligned(counts):
             want = q2.switch_glu_expert(x[row_tok[r]].astype(np.float64), *expert_fn(mlx)(u), bits=2, group=64)
             err = np.linalg.norm(got[row_out[r]].astype(np.float64) - want) / np.linalg.norm(want)
             assert err <= BOUND, (u, err)
+
+
+@pytest.mark.parametrize("hidden,inter", [(2048, 512), (2048, 576), (384, 512), (2560, 192), (320, 256)])
+@pytest.mark.parametrize("form", ["blob", "fp16", "bf16"])
+def test_same_bits_whatever_the_call(hidden, inter, form):
+    """At K = 2048 (gate/up) and K = 512 (down) the whole-K kernels take the calls with few rows per segment and
+    k_q2g_mm the others, in its several forms there and at every other K; a row's result does not depend on which:
+    all rows in one call, one call per segment and one-tile segments give the same bits, also with a last slice only
+    partly in range (inter 576, hidden 384)."""
+    from moe_offload import _lib, ops, prefill
+    dev = torch.device("cuda")
+    n_exp = 10
+    rng = np.random.default_rng(hidden + inter)
+    mlx, blobs = experts_np(n_exp, hidden, inter, seed=8)
+    if form == "bf16":
+        mlx = experts_bf16(n_exp, hidden, inter, seed=8)
+    counts = np.array([130, 40, 1, 16, 64, 17, 70, 31, 90, 15])
+    x = rng.standard_normal((50, hidden)).astype(np.float16)
+    row_tok, row_out, seg_start = _plan(counts, 50, rng)
+    seg_slot = rng.permutation(n_exp).astype(np.int32)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    pools = _pools(mlx, dev) if form != "blob" else None
+
+    def call(rt, ro, ss, sl):
+        if form == "blob":
+            out = torch.zeros((row_tok.size, hidden), dtype=torch.float16, device=dev)
+            return ops.q2_grouped_switch_glu(t(x), t(rt), t(ss), t(blobs), hidden, inter, row_out=t(ro),
+                                             n_out_rows=row_tok.size, seg_slot=t(sl), out=out).cpu().numpy()
+        return _grouped_t(_lib.lib(), t(x), t(rt), t(ro), t(ss), t(sl), pools[1], pools[2], int(form == "bf16"), n_exp,
+                          hidden, inter, row_tok.size)
+
+    want = call(row_tok, row_out, seg_start, seg_slot)          # 474 rows over 10 segments
+    tiles = prefill.tile_segments(seg_start, seg_slot)
+    assert np.array_equal(call(row_tok, row_out, *tiles), want)
+    for u in range(n_exp):
+        r = slice(int(seg_start[u]), int(seg_start[u + 1]))
+        got = call(row_tok[r], row_out[r], np.array([0, counts[u]], np.int32), seg_slot[u:u + 1])
+        assert np.array_equal(got[row_out[r]], want[row_out[r]]), (u, int(counts[u]))
+    _check(want, x, row_tok, row_out, seg_start, seg_slot, expert_fn(mlx), "bf16" if form == "bf16" else None)
