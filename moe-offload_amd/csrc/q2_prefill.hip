@@ -132,9 +132,10 @@ __device__ __forceinline__ void transpose4(uint32_t& a, uint32_t& b, uint32_t& c
 // These are k_q2g_mm's positions in k_q2g_mm's order, so a row's h has the same bits whichever of
 // the two kernels a call's size selects.  (The other way round, a quarter of K per lane group in
 // both, costs k_q2g_mm 25% at this K: each of its steps would touch every line of a weight row.)
-// The 9-tensor form's scales and biases still come in one 16-byte load each, a quarter of a row per
-// lane group, and are dealt out between the groups in registers: 512 tokens, top-10 of 512, 2048 x
-// 512 bf16: 178 us for gate/up + down + combine, 190 with a 4-byte load per pair of groups.
+// The scales and biases still come in 16-byte loads, a quarter of a row per lane group, and are dealt
+// out between the groups in registers: gate/up + down + combine of 512 tokens, top-10 of 512, 2048 x
+// 512: 176 us (bf16) against 190 with a 4-byte load per pair of groups; gate/up of one to four
+// blob segments 13.1 us against 13.9 with 8-byte loads.
 template <int GPL, int SBF>
 __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n_src_rows,
                                            const int32_t* __restrict__ row_map, int r0, int rows, int slot,
@@ -186,12 +187,14 @@ __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n
             for (int i = 0; i < GPL; ++i) c[h][i] = *reinterpret_cast<const uint4*>(cr + (i >> 1) * 128 + (i & 1) * 16);
             if constexpr (SBF == 0) {
                 const uint32_t* sr = reinterpret_cast<const uint32_t*>(P.s + (size_t)slot * P.s_stride) +
-                                     (size_t)(base + n) * kg + 2 * kq;
+                                     (size_t)(base + n) * kg + GPL * kq;
 #pragma unroll
-                for (int i = 0; i < GPL; i += 2) {
-                    const uint2 v = *reinterpret_cast<const uint2*>(sr + 4 * i);
-                    wd[h][i] = v.x;
-                    wd[h][i + 1] = v.y;
+                for (int i = 0; i < GPL / 4; ++i) {
+                    const uint4 v = reinterpret_cast<const uint4*>(sr)[i];
+                    wd[h][4 * i] = v.x;
+                    wd[h][4 * i + 1] = v.y;
+                    wd[h][4 * i + 2] = v.z;
+                    wd[h][4 * i + 3] = v.w;
                 }
             } else {
                 // groups 8kq .. 8kq + 7, two to a word: scales in the even elements, biases in the odd
@@ -211,10 +214,8 @@ __device__ __forceinline__ void gu_whole_k(const __half* __restrict__ src, int n
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
             for (int i = 0; i < GPL; ++i) w[h][i] = wd[h][i];
-            if constexpr (SBF != 0) {
-                transpose4(w[h][0], w[h][2], w[h][4], w[h][6]);
-                transpose4(w[h][1], w[h][3], w[h][5], w[h][7]);
-            }
+            transpose4(w[h][0], w[h][2], w[h][4], w[h][6]);
+            transpose4(w[h][1], w[h][3], w[h][5], w[h][7]);
         }
 #pragma unroll
         for (int i = 0; i < GPL; ++i) {
