@@ -990,14 +990,17 @@ template <int MODE, int SBF>
 int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row_map, const int32_t* row_out,
                     int n_out_rows, const int32_t* seg_start, const int32_t* seg_slot, int n_seg, int n_rows,
                     const Q2Experts& E, int n_slots, int hidden, int inter, __half* out, hipStream_t s) {
-    // Few rows per expert at the two shapes the whole-K kernels are built for: those, whose short
-    // blocks (512 or more, 2-4 per CU) hide each other's latencies; from about one full M tile per
-    // expert on, k_q2g_mm's one pass over the weights per 64 rows wins (gate/up + down + combine, 512
-    // experts of 2048 x 512: 16 tokens x top-10 40 us against 58, 128 tokens 115 against 145, 512
-    // tokens 186 against 191, 2048 tokens 540 against 350).  The line is drawn on the pool's slots,
-    // not on the segments, so cutting segments into pieces does not change the kernel (nor a bit of
-    // the result).
-    if (n_rows < 16LL * n_slots) {
+    // Short segments at the two shapes the whole-K kernels are built for: those, whose short blocks
+    // (512 or more, 2-4 per CU) hide each other's latencies; from about one full M tile per segment on,
+    // k_q2g_mm's one pass over the weights per 64 rows wins (gate/up + down + combine in us, whole-K
+    // against k_q2g_mm, 512 experts of 2048 x 512 and top-10: 64 tokens 88 and 97 at 4 of 512, 512 tokens
+    // 167 and 191, 1024 tokens 253 and 210, 2048 tokens 480 and 289; one segment of 16 rows 20.8 and
+    // 23.5, of 40 rows 51 and 28; 250 segments of 32 rows 262 and 137).  The line is drawn on the
+    // segments and not on the pool's slots: rows on a few experts of a large pool are long segments too,
+    // and a plan cut into one-tile segments keeps the kernel that is made for it (2048 tokens, gate/up
+    // over one-tile segments: 233 us whole-K, 266 in k_q2g_mm, which reads the weights once per segment).
+    // Both kernels give the same bits.
+    if (n_rows <= 16LL * n_seg) {
         if constexpr (MODE == kGateUp) {
             if (K == 2048)
                 return launch_gu_wk<SBF>(src, n_src_rows, row_map, seg_start, seg_slot, n_seg, n_rows, E, n_slots, inter,

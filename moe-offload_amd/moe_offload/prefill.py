@@ -147,13 +147,13 @@ def cached_prefill(module, x: torch.Tensor, indices: torch.Tensor) -> torch.Tens
 def tile_segments(seg_start: np.ndarray, seg_slot: np.ndarray, rows: int = 16):
     """The same sorted rows cut into segments of at most `rows` rows, each keeping its expert's slot.
 
-    For gate/up at hidden 2048 with fewer than 16 rows per slot of the pool (the whole-K form): that
-    kernel gives every (segment, 128-row slice) one block that takes the segment's 16-row M tiles one
-    after the other; an expert of several tiles given as several one-tile segments runs as
-    neighbouring blocks on one XCD instead, which read its weights together (from L2 after the first)
-    rather than one block re-reading them per tile.  Outputs are bit-identical (each tile is
-    multiplied the same way).  All other shapes multiply up to four tiles per weight pass and are
-    faster over the expert segments.  Empty segments are dropped.
+    For gate/up at hidden 2048 with at most 16 rows per expert (the whole-K form): that kernel gives
+    every (segment, 128-row slice) one block that takes the segment's 16-row M tiles one after the
+    other; an expert of several tiles given as several one-tile segments runs as neighbouring blocks
+    on one XCD instead, which read its weights together (from L2 after the first) rather than one
+    block re-reading them per tile.  With more rows per expert, and at all other shapes, the expert
+    segments are faster: the kernel there multiplies up to four tiles per weight pass.  Outputs are
+    bit-identical either way.  Empty segments are dropped.
     Returns int32 (seg_start', seg_slot').
     """
     seg_start = np.asarray(seg_start, dtype=np.int64)
