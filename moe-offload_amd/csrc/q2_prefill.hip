@@ -11,11 +11,12 @@
 // Tiling.  The rows of a segment form M tiles of 16 (v_mfma_f32_16x16x32_f16).  k_q2g_mm takes up to
 // 64 rows of a segment per pass over its weights, with their activations staged in LDS for the whole
 // K and, for all but short calls, a fixed grid whose blocks split the work evenly.  With few rows per
-// expert, K = 2048 gate/up and K = 512 down run in the whole-K forms: k_q2g_gu_wk (per M tile, each
-// wave's weight subtiles requested over the whole K at once, the tile's activations staged once) and
-// k_q2g_dn_wk (each wave's 4 subtiles loaded once and kept in registers while the segment's M tiles
-// pass through LDS), both with a grid that holds every (segment, slice) item twice: segments of
-// several tiles run in the first half, so their blocks, the longest, are dispatched before the rest.
+// expert the whole-K forms run: gate/up at K = 2048 in k_q2g_gu_wk (per M tile, each wave's weight
+// subtiles requested over the whole K at once, the tile's activations staged once), down at K = 512
+// and both up to K = 256 in k_q2g_wk (each wave's 4 subtiles loaded once and kept in registers while
+// the segment's M tiles pass through LDS).  All but the last with K <= 256 for down have a grid that
+// holds every (segment, slice) item twice: segments of several passes run in the first half, so their
+// blocks, the longest, are dispatched before the rest.
 //
 // Dequantisation.  A 2-bit code in the low bits of a nibble is the fp4 (e2m1) value q/2, so
 // w & 0x33333333 (even codes) and (w >> 2) & 0x33333333 (odd codes) are 8 fp4 values each;
@@ -799,22 +800,36 @@ __global__ __launch_bounds__(64 * WV, TM == 1 ? 4 : 2) void k_q2g_mm(
     }
 }
 
-// Down in the whole-K form (K = inter = 256 * GPL): a block takes one segment and 256 output rows,
-// each wave 4 subtiles of 16 rows whose whole K it requests at once and keeps in registers while
-// the segment's 16-row tiles of h pass through LDS (staged for the whole K, split into the MFMA's
-// even / odd fragments; one barrier per tile).  Output row r goes to row_out[r] (or r).  Lane group kq
-// takes groups 2kq and 2kq + 1: at K = 512 these are k_q2g_mm's positions, and the sums have its bits.
-template <int GPL, int SBF>
-__global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
-    const __half* __restrict__ src, int n_src_rows, const int32_t* __restrict__ row_out, int n_out_rows,
+// Short K in the whole-K form (K = 512, GPL 2; any K up to 256, GPL 1): a block takes one segment and 256
+// output rows (128 of each projection for gate/up), each wave 4 subtiles of 16 rows whose whole K it
+// requests at once and keeps in registers while the segment's rows pass through LDS (staged for the
+// whole K, split into the MFMA's even / odd fragments; one barrier per pass).  row_idx names each row's
+// source row (gate/up) or output row (down); without it they are the same.  Lane group kq takes groups
+// GPL*kq .. GPL*kq + GPL - 1: at K = 512 and up to 256 these are k_q2g_mm's positions, and the sums have
+// its bits.  Groups past a K below 256 read the last one; their activations are staged as zeros.
+//
+// What bounds it: one chain of dependent round trips per block (segment, rows, activations beside the
+// weights) and the dequantisation.  Up to K 256 k_q2g_mm leaves half of every 512-input step empty, and
+// its waves hold half as many weights; two M tiles per pass share the dequantisation.  Down in us, the
+// chunked kernel of old / k_q2g_mm / this: 137 tokens x top-10 of 280, 1728 x 256: 17.2 / 26 / 16.7; 79 x
+// top-5 of 66, 2304 x 256: 8.0 / 13.3 / 8.1; 222 x top-7 of 202, 512 x 256: 9.4 / 13.6 / 9.0; gate/up of
+// 924 x top-4 of 338, 256 x 576: 19.5 / 23.5 / 19.0.  One tile per pass: 1-3 us slower where segments
+// exceed 16 rows; 5 or 6 blocks per CU instead of 4: spills.
+template <int GPL, int MODE>
+constexpr bool two_pass() { return GPL == 2 || MODE == kGateUp; }
+
+template <int GPL, int MODE, int SBF>
+__global__ __launch_bounds__(256, 2) void k_q2g_wk(
+    const __half* __restrict__ src, int n_src_rows, const int32_t* __restrict__ row_idx, int n_out_rows,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_slot, int n_seg, int n_rows,
-    Q2Experts E, int n_slots, int hidden, int tiles_per_seg, __half* __restrict__ out) {
-    constexpr int K = 256 * GPL;
-    constexpr int kg = 4 * GPL;
-    constexpr int UPR = K / 8;                        // 16-byte units per h row
+    Q2Experts E, int n_slots, int N, int tiles_per_seg, __half* __restrict__ out, int k_len) {
+    const int K = GPL == 1 ? k_len : 256 * GPL, kg = K / 64;
+    constexpr int UPR = 32 * GPL;                     // 16-byte units per activation row in LDS
     constexpr int kPairsPerThread = UPR / 32;         // unit pairs a thread stages per tile
-    static_assert(kPairsPerThread >= 1, "K >= 256");
-    __shared__ uint4 a_lds[16 * UPR];
+    constexpr int NT = GPL == 1 ? 2 : 1;              // M tiles per pass
+    // segments of several passes first, in a grid of twice the items; a short K's down is as fast without
+    constexpr bool kTwoPass = two_pass<GPL, MODE>();
+    __shared__ uint4 a_lds[NT * 16 * UPR];
     const int items = n_seg * tiles_per_seg;
     const int pass = (int)blockIdx.x >= items ? 1 : 0;
     const int work = xcd_order((int)blockIdx.x - pass * items, items);
@@ -825,36 +840,35 @@ __global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
     r1 = r1 < r0 ? r0 : (r1 > n_rows ? n_rows : r1);
     const int slot = seg_slot ? seg_slot[seg] : seg;
     if (r1 == r0 || slot < 0 || slot >= n_slots) return;
-    if ((pass == 0) != (r1 - r0 > kMT)) return;       // segments of several tiles first
+    if (kTwoPass && (pass == 0) != (r1 - r0 > NT * kMT)) return;
 
     const int t0 = threadIdx.x, lane0 = t0 & 63, wv = __builtin_amdgcn_readfirstlane(t0 >> 6);
     const int n0 = lane0 & 15, kq0 = lane0 >> 4;
-    const Q2Proj& P = E.p[2];
+    const int g0 = GPL > 1 || kq0 < kg ? GPL * kq0 : kg - 1;
     const size_t code_row = (size_t)K / 4;
-    // the wave's 4 subtiles: output rows base_s .. base_s + 15 (hidden is a multiple of 64)
+    // the wave's 4 subtiles: rows base .. base + 15 of their projection (N is a multiple of 64)
     uint4 cw[4][GPL];
     uint32_t sw[4][GPL];
     bool rv[4];
     int col[4];
 #pragma unroll
     for (int sIdx = 0; sIdx < 4; ++sIdx) {
-        int base = tile * 256 + wv * 64 + sIdx * 16;
-        rv[sIdx] = base < hidden;
+        int base = MODE == kGateUp ? tile * 128 + wv * 32 + (sIdx >> 1) * 16 : tile * 256 + wv * 64 + sIdx * 16;
+        const Q2Proj& P = E.p[MODE == kGateUp ? (sIdx & 1) : 2];
+        rv[sIdx] = base < N;
         col[sIdx] = base + n0;
-        if (base >= hidden) base = hidden - 16;
-        const uint8_t* cr = P.w + (size_t)slot * P.w_stride + (size_t)(base + n0) * code_row + (size_t)(GPL * kq0) * 16;
+        if (base >= N) base = N - 16;
+        const uint8_t* cr = P.w + (size_t)slot * P.w_stride + (size_t)(base + n0) * code_row + (size_t)g0 * 16;
 #pragma unroll
         for (int i = 0; i < GPL; ++i) cw[sIdx][i] = *reinterpret_cast<const uint4*>(cr + (size_t)i * 16);
+        const size_t o = (size_t)(base + n0) * kg + g0;
         if constexpr (SBF == 0) {
-            const uint32_t* sr = reinterpret_cast<const uint32_t*>(P.s + (size_t)slot * P.s_stride) +
-                                 (size_t)(base + n0) * kg + GPL * kq0;
+            const uint32_t* sr = reinterpret_cast<const uint32_t*>(P.s + (size_t)slot * P.s_stride) + o;
 #pragma unroll
             for (int i = 0; i < GPL; ++i) sw[sIdx][i] = sr[i];
         } else {
-            const uint16_t* scr = reinterpret_cast<const uint16_t*>(P.s + (size_t)slot * P.s_stride) +
-                                  (size_t)(base + n0) * kg + GPL * kq0;
-            const uint16_t* bir = reinterpret_cast<const uint16_t*>(P.b + (size_t)slot * P.b_stride) +
-                                  (size_t)(base + n0) * kg + GPL * kq0;
+            const uint16_t* scr = reinterpret_cast<const uint16_t*>(P.s + (size_t)slot * P.s_stride) + o;
+            const uint16_t* bir = reinterpret_cast<const uint16_t*>(P.b + (size_t)slot * P.b_stride) + o;
 #pragma unroll
             for (int i = 0; i < GPL; ++i) sw[sIdx][i] = sb_word<SBF>(scr[i], bir[i]);
         }
@@ -863,41 +877,57 @@ __global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
 
     const int sm = t0 >> 4, sv0 = t0 & 15;
 #pragma unroll 1
-    for (int m0 = r0; m0 < r1; m0 += kMT) {          // block-uniform
-        const int rows_t = (r1 - m0) < kMT ? (r1 - m0) : kMT;
-        int srow = -1;
-        if (sm < rows_t) {
-            srow = m0 + sm;
-            if (srow >= n_src_rows) srow = -1;
-        }
-        uint4 xv[2 * kPairsPerThread];
-        const uint4* xr = reinterpret_cast<const uint4*>(src + (size_t)(srow < 0 ? 0 : srow) * K);
+    for (int m0 = r0; m0 < r1; m0 += NT * kMT) {     // block-uniform
+        const int rows_t = (r1 - m0) < NT * kMT ? (r1 - m0) : NT * kMT;
+        const bool two = NT > 1 && rows_t > kMT;
+        int srow[NT];
+        uint4 xv[NT][2 * kPairsPerThread];
 #pragma unroll
-        for (int c = 0; c < kPairsPerThread; ++c) {
-            xv[2 * c] = xr[2 * (sv0 + 16 * c)];
-            xv[2 * c + 1] = xr[2 * (sv0 + 16 * c) + 1];
-        }
-        if (m0 > r0) lds_barrier();                   // every wave is done with the last tile
+        for (int u = 0; u < NT; ++u) {
+            if (u && !two) break;
+            srow[u] = -1;
+            if (u * kMT + sm < rows_t) {
+                srow[u] = m0 + u * kMT + sm;
+                if (MODE == kGateUp && row_idx) srow[u] = row_idx[srow[u]];
+                if ((unsigned)srow[u] >= (unsigned)n_src_rows) srow[u] = -1;
+            }
+            const uint4* xr = reinterpret_cast<const uint4*>(src + (size_t)(srow[u] < 0 ? 0 : srow[u]) * K);
 #pragma unroll
-        for (int c = 0; c < kPairsPerThread; ++c) {
-            const int v = 2 * (sv0 + 16 * c);
-            f16x8 ev, od;
-            split_even_odd(xv[2 * c], xv[2 * c + 1], ev, od);
-            const uint4 e4 = __builtin_bit_cast(uint4, ev), o4 = __builtin_bit_cast(uint4, od);
-            a_lds[sm * UPR + (v ^ sm)] = srow >= 0 ? e4 : make_uint4(0, 0, 0, 0);
-            a_lds[sm * UPR + ((v + 1) ^ sm)] = srow >= 0 ? o4 : make_uint4(0, 0, 0, 0);
+            for (int c = 0; c < kPairsPerThread; ++c) {
+                const int pv = GPL == 1 && sv0 * 16 >= K ? 0 : sv0 + 16 * c;
+                xv[u][2 * c] = xr[2 * pv];
+                xv[u][2 * c + 1] = xr[2 * pv + 1];
+            }
+        }
+        if (m0 > r0) lds_barrier();                   // every wave is done with the last pass
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            if (u && !two) break;
+            const bool live = srow[u] >= 0 && (GPL > 1 || sv0 * 16 < K);
+            uint4* d = a_lds + (u * kMT + sm) * UPR;
+#pragma unroll
+            for (int c = 0; c < kPairsPerThread; ++c) {
+                const int v = 2 * (sv0 + 16 * c);
+                f16x8 ev, od;
+                split_even_odd(xv[u][2 * c], xv[u][2 * c + 1], ev, od);
+                const uint4 e4 = __builtin_bit_cast(uint4, ev), o4 = __builtin_bit_cast(uint4, od);
+                d[v ^ sm] = live ? e4 : make_uint4(0, 0, 0, 0);
+                d[(v + 1) ^ sm] = live ? o4 : make_uint4(0, 0, 0, 0);
+            }
         }
         lds_barrier();
-        // opaque per tile: the converted weights and the fragment addresses are not kept across
-        // tiles
+        // opaque per pass: the converted weights and the fragment addresses are not kept across
+        // passes
         uint32_t z;
         asm volatile("v_mov_b32 %0, 0" : "=v"(z));
         int tq = (int)threadIdx.x;
         asm volatile("" : "+v"(tq));
         const int n = tq & 15, kq = (tq & 63) >> 4;
-        f32x4 acc[4];
+        f32x4 acc[NT][4];
 #pragma unroll
-        for (int sIdx = 0; sIdx < 4; ++sIdx) acc[sIdx] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int sIdx = 0; sIdx < 4; ++sIdx) acc[u][sIdx] = (f32x4){0.f, 0.f, 0.f, 0.f};
         const uint4* arow = a_lds + n * UPR;
 #pragma unroll
         for (int i = 0; i < GPL; ++i) {
@@ -908,30 +938,51 @@ __global__ __launch_bounds__(256, 2) void k_q2g_dn_wk(
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int v = u0 + 2 * q;
-                const f16x8 a_ev = __builtin_bit_cast(f16x8, arow[v ^ n]);
-                const f16x8 a_od = __builtin_bit_cast(f16x8, arow[(v + 1) ^ n]);
+                f16x8 a_ev[NT], a_od[NT];
+#pragma unroll
+                for (int u = 0; u < NT; ++u) {
+                    if (u && !two) break;
+                    a_ev[u] = __builtin_bit_cast(f16x8, arow[u * kMT * UPR + (v ^ n)]);
+                    a_od[u] = __builtin_bit_cast(f16x8, arow[u * kMT * UPR + ((v + 1) ^ n)]);
+                }
 #pragma unroll
                 for (int sIdx = 0; sIdx < 4; ++sIdx) {
                     const uint4 cv = cw[sIdx][i];
                     const uint32_t wq = (q == 0 ? cv.x : q == 1 ? cv.y : q == 2 ? cv.z : cv.w) ^ z;
                     const f16x8 b_ev = dequant8(wq & 0x33333333u, sb[sIdx]);
                     const f16x8 b_od = dequant8((wq >> 2) & 0x33333333u, sb[sIdx]);
-                    acc[sIdx] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_ev, b_ev, acc[sIdx], 0, 0, 0);
-                    acc[sIdx] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_od, b_od, acc[sIdx], 0, 0, 0);
+#pragma unroll
+                    for (int u = 0; u < NT; ++u) {
+                        if (u && !two) break;
+                        acc[u][sIdx] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_ev[u], b_ev, acc[u][sIdx], 0, 0, 0);
+                        acc[u][sIdx] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_od[u], b_od, acc[u][sIdx], 0, 0, 0);
+                    }
                 }
             }
         }
         // lane holds rows 4 kq + i of column n of each subtile
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = 4 * kq + i;
-            if (m >= rows_t) continue;
-            const int r = m0 + m;
-            const int orow = row_out ? row_out[r] : r;
-            if (orow < 0 || orow >= n_out_rows) continue;
+        for (int u = 0; u < NT; ++u) {
+            if (u && !two) break;
 #pragma unroll
-            for (int sIdx = 0; sIdx < 4; ++sIdx)
-                if (rv[sIdx]) out[(size_t)orow * hidden + col[sIdx]] = __float2half_rn(acc[sIdx][i]);
+            for (int i = 0; i < 4; ++i) {
+                const int m = u * kMT + 4 * kq + i;
+                if (m >= rows_t) continue;
+                const int r = m0 + m;
+                if constexpr (MODE == kGateUp) {
+#pragma unroll
+                    for (int sIdx = 0; sIdx < 4; sIdx += 2) {
+                        const float g = acc[u][sIdx][i], up = acc[u][sIdx + 1][i];
+                        if (rv[sIdx]) out[(size_t)r * N + col[sIdx]] = __float2half_rn(g / (1.0f + __expf(-g)) * up);
+                    }
+                } else {
+                    const int orow = row_idx ? row_idx[r] : r;
+                    if (orow < 0 || orow >= n_out_rows) continue;
+#pragma unroll
+                    for (int sIdx = 0; sIdx < 4; ++sIdx)
+                        if (rv[sIdx]) out[(size_t)orow * N + col[sIdx]] = __float2half_rn(acc[u][sIdx][i]);
+                }
+            }
         }
     }
 }
@@ -973,15 +1024,16 @@ int launch_gu_wk(const __half* src, int n_src_rows, const int32_t* row_map, cons
     return 0;
 }
 
-template <int SBF>
-int launch_dn_wk(const __half* src, int n_src_rows, const int32_t* row_out, int n_out_rows, const int32_t* seg_start,
-                 const int32_t* seg_slot, int n_seg, int n_rows, const Q2Experts& E, int n_slots, int hidden,
-                 __half* out, hipStream_t s) {
-    const int tiles = (hidden + 255) / 256;
-    const long long nb = 2LL * n_seg * tiles;                  // two passes
+template <int GPL, int MODE, int SBF>
+int launch_wk(int K, const __half* src, int n_src_rows, const int32_t* row_map, const int32_t* row_out, int n_out_rows,
+              const int32_t* seg_start, const int32_t* seg_slot, int n_seg, int n_rows, const Q2Experts& E, int n_slots,
+              int N, __half* out, hipStream_t s) {
+    const int tiles = MODE == kGateUp ? (N + 127) / 128 : (N + 255) / 256;
+    const long long nb = (two_pass<GPL, MODE>() ? 2LL : 1LL) * n_seg * tiles;
     if (nb > 0x7FFFFFFFLL) { moe_set_error("grouped q2: grid too large"); return -1; }
-    MOE_LAUNCH(TK_PF_DOWN, (k_q2g_dn_wk<2, SBF>), dim3((unsigned)nb), dim3(256), 0, s, src, n_src_rows, row_out,
-               n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots, hidden, tiles, out);
+    MOE_LAUNCH(MODE == kGateUp ? TK_PF_GATE_UP : TK_PF_DOWN, (k_q2g_wk<GPL, MODE, SBF>), dim3((unsigned)nb), dim3(256), 0,
+               s, src, n_src_rows, MODE == kGateUp ? row_map : row_out, n_out_rows, seg_start, seg_slot, n_seg, n_rows, E,
+               n_slots, N, tiles, out, K);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -1006,19 +1058,39 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
                 return launch_gu_wk<SBF>(src, n_src_rows, row_map, seg_start, seg_slot, n_seg, n_rows, E, n_slots, inter,
                                          out, s);
         } else if (K == 512) {
-            return launch_dn_wk<SBF>(src, n_src_rows, row_out, n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots,
-                                     hidden, out, s);
+            return launch_wk<2, MODE, SBF>(K, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg,
+                                           n_rows, E, n_slots, hidden, out, s);
         }
+    }
+    const int N = MODE == kGateUp ? inter : hidden;
+    const long long t4 = (N + (MODE == kGateUp ? 63 : 127)) / (MODE == kGateUp ? 64 : 128), t8 = (t4 + 1) / 2;
+    // K up to 256: the whole-K form while the segments are short; the longest one sets its time, so the
+    // line lies lower with few column tiles, whose other work is soon done.  Whole-K against k_q2g_mm in
+    // us: 300 segments of 14 rows, down to 2304 x 256: 26 and 35, of 30 rows 42 and 41; 100 of 14 rows to
+    // 1024 x 128: 10.4 and 12.1, of 30 rows 17.0 and 13.9; 133 of 17 rows to 512 x 192: 16.0 and 9.8; gate/up
+    // of 300 segments of 20 rows, 256 x 512: 20.4 and 25; 8 segments of 20 rows, 128 x 256: 5.7 and 7.5.
+    // The smallest down products stay with k_q2g_mm's one-segment blocks, which start sooner (4.6-4.7 us
+    // against 5.0).
+    if (K <= 256) {
+        const int most_rows = K > 128 ? K / 8 : 16, by_tiles = MODE == kGateUp ? N / 16 : N / 64;
+        long long line = by_tiles < most_rows ? by_tiles : most_rows;
+        const int least = MODE == kDown && K <= 192 ? 8 : 12;
+        if (line < least) line = least;
+        if (n_seg <= 16 && n_rows <= 256) line = 32;
+        const long long tiny = n_seg <= 16 ? 16 : n_seg <= 32 ? 8 : 4;
+        const bool smallest = MODE == kDown && n_seg * t4 <= kCUs && n_rows <= tiny * n_seg;
+        if (n_rows <= line * n_seg && !smallest)
+            return launch_wk<1, MODE, SBF>(K, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg,
+                                           n_rows, E, n_slots, N, out, s);
     }
     auto go = [&](auto tm, auto wv, int span) {
         return launch_mm<MODE, SBF, decltype(tm)::value, decltype(wv)::value>(
             K, span, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots,
-            MODE == kGateUp ? inter : hidden, out, s);
+            N, out, s);
     };
     using One = std::integral_constant<int, 1>;
     using Four = std::integral_constant<int, 4>;
     using Eight = std::integral_constant<int, 8>;
-    const int N = MODE == kGateUp ? inter : hidden;
     // Short calls: blocks of one segment and a few column tiles instead of shares, so that no block starts
     // with the sum over the segments (2-3 us), while the blocks are few and the segments short; K up
     // to 1024 in blocks of 4 waves, four per CU.  Gate/up + down + combine in us (chunked kernel
@@ -1027,7 +1099,6 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
     // lie where the shares win again: 415 x top-6 of 289, 960 x 512 (8.6 rows per expert) 61.3
     // against 63.4; 54 x top-8 of 95, 1216 x 448 (4.5 rows) 34.0 against 39.3; 64 x top-10 of 512,
     // 2560 x 640 (367 segments, 1,835 blocks) 152 against 175.
-    const long long t4 = (N + (MODE == kGateUp ? 63 : 127)) / (MODE == kGateUp ? 64 : 128), t8 = (t4 + 1) / 2;
     // A block takes as many column tiles as keep the grid at 2,048 blocks, 1,024 with the shortest
     // segments (55 x top-3 of 401, 2240 x 256: 36.6 against 34.0; 415 x top-6 of 289: 65.7 against 75.3).
     const long long most = n_rows <= 4LL * n_seg ? 1024 : 2048;

@@ -118,13 +118,14 @@ def test_mm_out_of_range_and_unaligned(counts):
             assert err <= BOUND, (u, err)
 
 
-@pytest.mark.parametrize("hidden,inter", [(2048, 512), (2048, 576), (384, 512), (2560, 192), (320, 256)])
+@pytest.mark.parametrize("hidden,inter", [(2048, 512), (2048, 576), (384, 512), (2560, 192), (320, 256), (192, 128),
+                                          (64, 64)])
 @pytest.mark.parametrize("form", ["blob", "fp16", "bf16"])
 def test_same_bits_whatever_the_call(hidden, inter, form):
-    """At K = 2048 (gate/up) and K = 512 (down) the whole-K kernels take the calls with few rows per segment and
-    k_q2g_mm the others, in its several forms there and at every other K; a row's result does not depend on which:
-    all rows in one call, one call per segment and one-tile segments give the same bits, also with a last slice only
-    partly in range (inter 576, hidden 384)."""
+    """At K = 2048 (gate/up), K = 512 (down) and up to K = 256 the whole-K kernels take the calls with few rows per
+    segment and k_q2g_mm the others, in its several forms there and at every other K; a row's result does not depend
+    on which: all rows in one call, one call per segment and one-tile segments give the same bits, also with a last
+    slice only partly in range (inter 576, hidden 384, 320 and 192)."""
     from moe_offload import _lib, ops, prefill
     dev = torch.device("cuda")
     n_exp = 10
