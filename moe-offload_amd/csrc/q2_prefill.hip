@@ -12,8 +12,8 @@
 // 64 rows of a segment per pass over its weights, with their activations staged in LDS for the whole
 // K and, for all but short calls, a fixed grid whose blocks split the work evenly.  With few rows per
 // expert the whole-K forms run: gate/up at K = 2048 in k_q2g_gu_wk (per M tile, each wave's weight
-// subtiles requested over the whole K at once, the tile's activations staged once), down at K = 512
-// and both up to K = 256 in k_q2g_wk (each wave's 4 subtiles loaded once and kept in registers while
+// subtiles requested over the whole K at once, the tile's activations staged once), both products at
+// K = 512 and up to K = 256 in k_q2g_wk (each wave's 4 subtiles loaded once and kept in registers while
 // the segment's M tiles pass through LDS).  All but the last with K <= 256 for down have a grid that
 // holds every (segment, slice) item twice: segments of several passes run in the first half, so their
 // blocks, the longest, are dispatched before the rest.
@@ -1083,6 +1083,16 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
             return launch_wk<1, MODE, SBF>(K, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg,
                                            n_rows, E, n_slots, N, out, s);
     }
+    // Gate/up at K 512 likewise, while its blocks hide each other's latencies: the more there are, the longer
+    // the segments may be.  Whole-K against k_q2g_mm in us: 255 segments of 4.3 rows, 512 x 512: 20.3 and
+    // 23.4; 278 of 5 rows to 768: 23.3 and 28.9; 277 of 13 rows to 320: 25.0 and 26.3; 107 of 12 rows to 384: 18.1
+    // and 14.1; 75 of 5 rows to 128: 7.1 and 6.2; 278 of 3.4 rows to 64: 11.2 and 7.3.
+    if (MODE == kGateUp && K == 512 && N >= 128 && n_seg * t4 > kCUs) {
+        const long long line = n_seg * t4 / 64 < 16 ? n_seg * t4 / 64 : 16;
+        if (n_rows <= line * n_seg)
+            return launch_wk<2, MODE, SBF>(K, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg,
+                                           n_rows, E, n_slots, N, out, s);
+    }
     auto go = [&](auto tm, auto wv, int span) {
         return launch_mm<MODE, SBF, decltype(tm)::value, decltype(wv)::value>(
             K, span, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg, n_rows, E, n_slots,
@@ -1096,19 +1106,29 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
     // to 1024 in blocks of 4 waves, four per CU.  Gate/up + down + combine in us (chunked kernel
     // before; shares; these): 12 tokens x top-7 of 28 experts, 512 x 256: 13.8, 19.2, 11.7; 251 x
     // top-4 of 381, 576 x 512: 45.5, 44.9, 40.4; 5 x top-7, 2176 x 576: 36.8, 33.7, 29.5.  The lines
-    // lie where the shares win again: 415 x top-6 of 289, 960 x 512 (8.6 rows per expert) 61.3
-    // against 63.4; 54 x top-8 of 95, 1216 x 448 (4.5 rows) 34.0 against 39.3; 64 x top-10 of 512,
-    // 2560 x 640 (367 segments, 1,835 blocks) 152 against 175.
+    // lie where the shares win again.  Gate/up, these and shares: 427 segments of 8.4 rows, 1024 x 320, 51
+    // and 41; 308 of 7.4 rows, 832 x 704, 51 and 46; 253 of 5.7 rows, 640 x 192, 15.4 and 20.9; 174 of 9.8
+    // rows, 704 x 320, 20.7 and 22.0; 8 of 20 rows, 1024 x 128, 10.3 and 10.8 (64-row batches 13.7).
     // A block takes as many column tiles as keep the grid at 2,048 blocks, 1,024 with the shortest
     // segments (55 x top-3 of 401, 2240 x 256: 36.6 against 34.0; 415 x top-6 of 289: 65.7 against 75.3).
     const long long most = n_rows <= 4LL * n_seg ? 1024 : 2048;
-    if (K <= 1024 && n_rows <= (n_rows <= 1024 ? 16LL : 10LL) * n_seg && n_seg * t4 <= 6144)
+    const long long short_rows = n_rows <= 256 ? 32 : n_rows <= 1024 ? 16 : n_seg * t4 > 2048 ? 7 : 10;
+    if (K <= 1024 && n_rows <= short_rows * n_seg && n_seg * t4 <= 6144)
         return go(One(), Four(), (int)((n_seg * t4 + most - 1) / most));
-    if (K > 1024 && n_rows <= 4LL * n_seg && n_seg * t8 <= 1024) return go(One(), Eight(), 1);
+    // Above K 1024, blocks of 8 waves.  54 x top-8 of 95, 1216 x 448 (4.5 rows): shares 34.0 against 39.3; 64 x
+    // top-10 of 512, 2560 x 640 (367 segments, 1,835 blocks) 152 against 175.  Grids that leave CUs idle
+    // wait for their longest segment, unless all are short (gate/up, these and shares: 208 blocks for 762
+    // rows, 1856 x 128, 26.2 and 18.4; 200 for 320, 1280 x 192, 14.8 and 13.4; 108 for 280, 1600 x 64, 12.2 and
+    // 14.1).
+    if (K > 1024 && n_rows <= 4LL * n_seg && n_seg * t8 <= 1024 && (n_rows <= 300 || n_seg * t8 >= kCUs))
+        return go(One(), Eight(), 1);
     // One-tile batches, two blocks per CU, for few rows per segment (256 tokens at 2560 x 640, 5 per
     // expert: 242 / 230 us against 246 / 232 with 64-row batches; 512 tokens, 10 per expert: 297 /
-    // 286 against 296 / 275) and for small work (1,660 x top-2 of 28, 256 x 512: 27.0 against 35.1).
-    if (n_rows <= 8LL * n_seg || (K <= 512 && n_rows <= 4096)) return go(One(), Eight(), 0);
+    // 286 against 296 / 275; up to K 1024 gate/up of 439 segments of 8.5 rows, 896 x 768, 64.5 against 70.6)
+    // and for small work (1,660 x top-2 of 28, 256 x 512: 27.0 against 35.1; but down of 1,020 rows over 22
+    // experts to 2304 x 256: 17.1 against 12.0).
+    const bool small_work = K <= 512 && n_rows <= 4096 && (MODE == kGateUp || (long long)n_rows * N <= 2000000);
+    if (n_rows <= (K <= 1024 ? 10LL : 8LL) * n_seg || small_work) return go(One(), Eight(), 0);
     return go(std::integral_constant<int, kMaxTiles>(), Eight(), 0);
 }
 

@@ -83,6 +83,10 @@ def test_mm_many_segments(hidden, inter):
     order = np.argsort(slot_of, kind="stable")               # one oracle call per slot
     starts = np.searchsorted(slot_of[order], np.arange(7))
     _check(y, x, row_tok[order], row_out[order], starts, np.arange(6), expert_fn(mlx))
+    # the same rows as six long segments: other kernels, the same bits
+    y6 = ops.q2_grouped_switch_glu(t(x), t(row_tok[order]), t(starts.astype(np.int32)), t(blobs), hidden, inter,
+                                   row_out=t(row_out[order]), n_out_rows=row_tok.size).cpu().numpy()
+    assert np.array_equal(y6, y)
 
 
 @pytest.mark.parametrize("counts", [LONG, SHORT], ids=["long", "short"])
