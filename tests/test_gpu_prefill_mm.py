@@ -5,10 +5,11 @@ error of at most 2^-11 each, so the 2-norm of a segment's error is within 3 * 2^
 * contraction lengths with one group, a last step of one half (at most 4 groups) and of two clamped
   halves, whole steps, and the longest (2560); segments of 0, 1, 16, 17, 64, 65 and 130 rows; blob
   pools and the 9-tensor form with fp16 and bf16 scales; output columns below and above one tile;
-* more segments than threads in a block, over a pool of few slots, with long and empty ones mixed in;
+* more segments than threads in a block, over a pool of few slots, with long and empty ones mixed in; blocks that
+  take several column tiles of a segment, shares in 64-row batches, more than 4096 rows of a short contraction;
 * the same rows in calls of different sizes, which select different kernels, give the same bits;
 * an output that starts 2 bytes past a 16-byte boundary, and rows that name no source row, no output
-  row and no slot, are handled as by the other kernels.
+  row and no slot, are handled alike in k_q2g_mm and, with short segments, the whole-K kernels.
 """
 import numpy as np
 import pytest
@@ -64,18 +65,32 @@ def test_mm_matches_oracle(hidden, inter, form, counts):
     _check(y, x, row_tok, row_out, seg_start, seg_slot, expert_fn(mlx), "bf16" if form == "bf16" else None)
 
 
-@pytest.mark.parametrize("hidden,inter", [(512, 128), (1088, 256)])
-def test_mm_many_segments(hidden, inter):
+def _few_rows():
+    counts = np.random.default_rng(7).integers(0, 4, 1300)
+    counts[[5, 700, 1299]] = [150, 64, 33]
+    counts[100:180] = 0
+    return counts
+
+
+@pytest.mark.parametrize("hidden,inter,counts", [
+    (512, 128, _few_rows()), (1088, 256, _few_rows()),
+    # one block per segment and 3 of 16 column tiles (gate/up), for segments of one and two batches
+    (640, 1024, np.random.default_rng(8).integers(1, 12, 300) + 12 * (np.arange(300) % 40 == 7)),
+    # shares over more segments than a block has threads, 64-row batches (gate/up)
+    (1088, 128, np.random.default_rng(9).integers(2, 20, 600)),
+    # the same with few long segments, at a K of part of a step and of one whole step
+    (320, 512, np.array([900, 0, 1200, 63, 700, 1500, 1, 65])),
+    (512, 320, np.array([900, 0, 1200, 63, 700, 1500, 1, 65])),
+], ids=["many_512", "many_1088", "span_640", "shares_1088", "long_320", "long_512"])
+def test_mm_many_segments(hidden, inter, counts):
     from moe_offload import ops
     dev = torch.device("cuda")
     rng = np.random.default_rng(7)
-    counts = rng.integers(0, 4, 1300)
-    counts[[5, 700, 1299]] = [150, 64, 33]
-    counts[100:180] = 0
+    n_seg = counts.size
     mlx, blobs = experts_np(6, hidden, inter, seed=5)
     x = rng.standard_normal((60, hidden)).astype(np.float16)
     row_tok, row_out, seg_start = _plan(counts, 60, rng)
-    seg_slot = rng.integers(0, 6, 1300).astype(np.int32)
+    seg_slot = rng.integers(0, 6, n_seg).astype(np.int32)
     t = lambda a: torch.from_numpy(a).to(dev)
     y = ops.q2_grouped_switch_glu(t(x), t(row_tok), t(seg_start), t(blobs), hidden, inter, row_out=t(row_out),
                                   n_out_rows=row_tok.size, seg_slot=t(seg_slot)).cpu().numpy()
@@ -89,11 +104,12 @@ def test_mm_many_segments(hidden, inter):
     assert np.array_equal(y6, y)
 
 
+@pytest.mark.parametrize("hidden,inter", [(320, 192), (192, 320), (2048, 512)])
 @pytest.mark.parametrize("counts", [LONG, SHORT], ids=["long", "short"])
-def test_mm_out_of_range_and_unaligned(counts):
+def test_mm_out_of_range_and_unaligned(counts, hidden, inter):
     from moe_offload import ops
     dev = torch.device("cuda")
-    hidden, inter, n_exp = 320, 192, len(counts)
+    n_exp = len(counts)
     rng = np.random.default_rng(9)
     mlx, blobs = experts_np(n_exp, hidden, inter, seed=6)
     x = rng.standard_normal((30, hidden)).astype(np.float16)

@@ -224,9 +224,11 @@ def _grouped_t(L, x, row_tok, row_out, seg_start, seg_slot, ptrs, nbytes, bf16, 
     return y.cpu().numpy()
 
 
-def test_grouped_tensor_form_equals_blob_kernels():
+@pytest.mark.parametrize("n_tok", [256, 64])
+def test_grouped_tensor_form_equals_blob_kernels(n_tok):
     """fp16 scales: the 9-tensor grouped path loads the same (scale, bias) values as the blob path
-    and gives bit-identical outputs (512 tokens x top-10 of 64 experts, hidden 2048 / inter 512)."""
+    and gives bit-identical outputs (hidden 2048 / inter 512, top-10 of 64 experts: 40 rows per segment
+    in k_q2g_mm, 10 in the whole-K kernels)."""
     from moe_offload import _lib, ops, prefill, q2format, synth
     L = _lib.lib()
     dev = torch.device("cuda")
@@ -234,8 +236,8 @@ def test_grouped_tensor_form_equals_blob_kernels():
     gate, up, down = synth.q2_experts(E, H, I, seed=21)
     pool = torch.from_numpy(q2format.to_blobs(gate, up, down, H, I)).to(dev)
     ts, ptrs, nbytes = _pools((gate, up, down), dev)
-    ids, _ = synth.prefill_routing(256, K, E)
-    xs = synth.hidden_states(256, H, seed=22)
+    ids, _ = synth.prefill_routing(n_tok, K, E)
+    xs = synth.hidden_states(n_tok, H, seed=22)
     row_tok, row_out, seg_start, seg_slot = prefill.resident_plan(ids, K)
     t = lambda a: torch.from_numpy(a).to(dev)
     want = ops.q2_grouped_switch_glu(t(xs), t(row_tok), t(seg_start), pool, H, I, row_out=t(row_out),
