@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256, 2) void k_q2g_gu_wk(
 // wave).  With span 0 a fixed grid (one block per CU at TM 4, two at TM 1) sums the items' costs
 // over the segments, and each block takes its own equal part of them in the order (segment, batch,
 // column tile), so neither a long segment nor the last round of blocks leaves CUs idle (777 tokens
-// over 100 experts of 1152 x 320: 118 -> 55 us, where one block used to take a 140-row segment in
+// over 100 experts of 1152 x 320: 118 -> 54 us, where one block used to take a 140-row segment in
 // five passes of dependent round trips).  With span > 0 a block is one segment and `span` column tiles.
 //
 // A block stages a batch's activations once, for the whole K (split into even / odd fragments), and
@@ -332,11 +332,14 @@ __global__ __launch_bounds__(256, 2) void k_q2g_gu_wk(
 //
 // What bounds it: the dequantisation (19 VALU operations per 16 weights and lane, about 83 cycles
 // against 33 of matrix unit per M tile).  Every weight is dequantised once per batch, so 64-row
-// batches where they fit.  512 tokens, top-10 of 512 experts at 2560 x 640 bf16: gate/up 161 us (524
-// MB, 3.3 TB/s; VALU issuing 56% of the time), down 102 us; 2048 tokens: 313 and 171 us.  Both and the
-// combine: 287 -> 241 us and 590 -> 430 us against the chunk-by-chunk kernel this replaced (32 rows per
-// pass).  Two subtile pairs per wave (256-column tiles, 2.5 of them at 640): 211 and 136 us; 12 waves
-// per block: 188 and 111; phase 0 of a half built under the half before: 157 and 106.
+// batches where they fit.  Timed passes of 2560 x 640 bf16, top-10 of 512 experts (gate/up + down +
+// combine, back to back), the chunk-by-chunk kernel this replaced (32 rows per pass) -> this: 37 tokens
+// 126 -> 115 us, 512 tokens 287 -> 242, 2048 tokens 590 -> 427.  Per launch under the profiler, which slows
+// both sides: 512 tokens gate/up 218 -> 168 us (524 MB of weights; VALU issuing 56% of the time), down 107
+// -> 109 (no gain, nor at 37 tokens); 2048 tokens 411 -> 306 and 225 -> 170.  Tried and not kept, 512
+// tokens, gate/up and down, in one session where this ran 161 and 102: two subtile pairs per wave
+// (256-column tiles, 2.5 of them at 640) 211 and 136; 12 waves per block 188 and 111; phase 0 of a half
+// built under the half before 157 and 106.
 constexpr int kMaxTiles = 4;                             // M tiles per batch, at most
 constexpr int kMmSubs = 2;                               // 16-row weight subtiles per wave
 constexpr int kCUs = 256;
