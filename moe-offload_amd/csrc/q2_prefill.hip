@@ -33,7 +33,6 @@
 // fp16 is exact for the normal range of fp16).
 #include <hip/hip_fp16.h>
 
-#include <cstdlib>
 #include <type_traits>
 
 #include "moe_common.h"
@@ -1045,6 +1044,10 @@ template <int MODE, int SBF>
 int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row_map, const int32_t* row_out,
                     int n_out_rows, const int32_t* seg_start, const int32_t* seg_slot, int n_seg, int n_rows,
                     const Q2Experts& E, int n_slots, int hidden, int inter, __half* out, hipStream_t s) {
+    // column tiles of 4 and of 8 waves; the whole-K grids (at most twice n_seg * t4 blocks) fit in 31 bits
+    const int N = MODE == kGateUp ? inter : hidden;
+    const long long t4 = (N + (MODE == kGateUp ? 63 : 127)) / (MODE == kGateUp ? 64 : 128), t8 = (t4 + 1) / 2;
+    const bool wk_fits = n_seg * t4 <= 0x3FFFFFFF;
     // Short segments at the two shapes the whole-K kernels are built for: those, whose short blocks
     // (512 or more, 2-4 per CU) hide each other's latencies; from about one full M tile per segment on,
     // k_q2g_mm's one pass over the weights per 64 rows wins (gate/up + down + combine in us, whole-K
@@ -1055,7 +1058,7 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
     // and a plan cut into one-tile segments keeps the kernel that is made for it (2048 tokens, gate/up
     // over one-tile segments: 233 us whole-K, 266 in k_q2g_mm, which reads the weights once per segment).
     // Both kernels give the same bits.
-    if (n_rows <= 16LL * n_seg) {
+    if (wk_fits && n_rows <= 16LL * n_seg) {
         if constexpr (MODE == kGateUp) {
             if (K == 2048)
                 return launch_gu_wk<SBF>(src, n_src_rows, row_map, seg_start, seg_slot, n_seg, n_rows, E, n_slots, inter,
@@ -1065,8 +1068,6 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
                                            n_rows, E, n_slots, hidden, out, s);
         }
     }
-    const int N = MODE == kGateUp ? inter : hidden;
-    const long long t4 = (N + (MODE == kGateUp ? 63 : 127)) / (MODE == kGateUp ? 64 : 128), t8 = (t4 + 1) / 2;
     // K up to 256: the whole-K form while the segments are short; the longest one sets its time, so the
     // line lies lower with few column tiles, whose other work is soon done.  Whole-K against k_q2g_mm in
     // us: 300 segments of 14 rows, down to 2304 x 256: 26 and 35, of 30 rows 42 and 41; 100 of 14 rows to
@@ -1074,7 +1075,7 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
     // of 300 segments of 20 rows, 256 x 512: 20.4 and 25; 8 segments of 20 rows, 128 x 256: 5.7 and 7.5.
     // The smallest down products stay with k_q2g_mm's one-segment blocks, which start sooner (4.6-4.7 us
     // against 5.0).
-    if (K <= 256) {
+    if (K <= 256 && wk_fits) {
         const int most_rows = K > 128 ? K / 8 : 16, by_tiles = MODE == kGateUp ? N / 16 : N / 64;
         long long line = by_tiles < most_rows ? by_tiles : most_rows;
         const int least = MODE == kDown && K <= 192 ? 8 : 12;
@@ -1090,7 +1091,7 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
     // the segments may be.  Whole-K against k_q2g_mm in us: 255 segments of 4.3 rows, 512 x 512: 20.3 and
     // 23.4; 278 of 5 rows to 768: 23.3 and 28.9; 277 of 13 rows to 320: 25.0 and 26.3; 107 of 12 rows to 384: 18.1
     // and 14.1; 75 of 5 rows to 128: 7.1 and 6.2; 278 of 3.4 rows to 64: 11.2 and 7.3.
-    if (MODE == kGateUp && K == 512 && N >= 128 && n_seg * t4 > kCUs) {
+    if (MODE == kGateUp && K == 512 && N >= 128 && n_seg * t4 > kCUs && wk_fits) {
         const long long line = n_seg * t4 / 64 < 16 ? n_seg * t4 / 64 : 16;
         if (n_rows <= line * n_seg)
             return launch_wk<2, MODE, SBF>(K, src, n_src_rows, row_map, row_out, n_out_rows, seg_start, seg_slot, n_seg,
