@@ -1051,9 +1051,9 @@ int dispatch_proj_f(int K, const __half* src, int n_src_rows, const int32_t* row
     // Short segments at the two shapes the whole-K kernels are built for: those, whose short blocks
     // (512 or more, 2-4 per CU) hide each other's latencies; from about one full M tile per segment on,
     // k_q2g_mm's one pass over the weights per 64 rows wins (gate/up + down + combine in us, whole-K
-    // against k_q2g_mm, 512 experts of 2048 x 512 and top-10: 64 tokens 88 and 97 at 4 of 512, 512 tokens
-    // 167 and 191, 1024 tokens 253 and 210, 2048 tokens 480 and 289; one segment of 16 rows 20.8 and
-    // 23.5, of 40 rows 51 and 28; 250 segments of 32 rows 262 and 137).  The line is drawn on the
+    // against k_q2g_mm, top-4 of 512 experts of 2048 x 512: 128 tokens 78 and 97, 512 tokens 125 and 144,
+    // 1024 tokens 157 and 159, 1536 tokens 190 and 170, 3584 tokens 426 and 240; one segment of 16 rows 20.8
+    // and 23.5, of 40 rows 51 and 28; 250 segments of 28 rows 262 and 137).  The line is drawn on the
     // segments and not on the pool's slots: rows on a few experts of a large pool are long segments too,
     // and a plan cut into one-tile segments keeps the kernel that is made for it (2048 tokens, gate/up
     // over one-tile segments: 233 us whole-K, 266 in k_q2g_mm, which reads the weights once per segment).
